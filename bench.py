@@ -9,8 +9,8 @@ One step = one full adjoint (k-space [coil][sample] in the caller's order in
 HBM -> coil-combined image) plus one full forward (image -> k-space) through
 the C ABI, everything resident in HBM. value = 2*M*C / step time.
 
-roofline: the adjoint gridding stage (spread_lane_kernel, reduce_chunks_kernel,
-fold_kernel: samples in HBM -> grid in HBM), algorithmic bytes per launch
+roofline: the adjoint gridding stage (tile_spread_kernel, tile_reduce_kernel:
+samples in HBM -> grid in HBM), algorithmic bytes per launch
 8*M*C + 4*d*M + 4*M (density) + 8*Ng*C, over the stage's average time
 measured with HIP events on the launch stream (library stage timer).
 cpu_baseline: the oracle restatement running the same adjoint + forward
@@ -80,7 +80,8 @@ def parse():
 
 
 # sources whose kernels the traffic counters measured
-TRAFFIC_SOURCES = ["gpunufft_amd/csrc/hip/gridding.hip", "gpunufft_amd/csrc/hip/gnufft_internal.hpp"]
+TRAFFIC_SOURCES = ["gpunufft_amd/csrc/hip/spread.hip", "gpunufft_amd/csrc/hip/gridding.hip",
+                   "gpunufft_amd/csrc/hip/gnufft_internal.hpp"]
 
 
 def sources_sha256():
@@ -107,7 +108,7 @@ def traffic_summary():
     return t
 
 
-GRIDDING_KERNELS = ("spread", "reduce", "fold", "interp")
+GRIDDING_KERNELS = ("tile_spread", "tile_reduce", "interp")
 
 
 def summarize_counters(paths, sha=None):
@@ -128,6 +129,7 @@ def summarize_counters(paths, sha=None):
             for r in csv.DictReader(f):
                 name = r["Kernel_Name"]
                 base = name[5:] if name.startswith("void ") else name
+                base = base.replace("(anonymous namespace)::", "")
                 key = None
                 for k in GRIDDING_KERNELS:
                     if base.startswith("gnufft::%s" % k) and "batch" not in base:
@@ -152,8 +154,7 @@ def summarize_counters(paths, sha=None):
         if "WRITE_SIZE" in e and "WRITE_SIZE" in cal:
             e["write_bytes"] = e["WRITE_SIZE"] * 1024.0 * cal["WRITE_SIZE"]
         kernels[k] = e
-    adj = [k for k in kernels if k.split("<")[0] in ("spread_lane_kernel", "spread_kernel",
-                                                      "reduce_chunks_kernel", "fold_kernel")]
+    adj = [k for k in kernels if k.split("<")[0] in ("tile_spread_kernel", "tile_reduce_kernel")]
     hbm = sum(kernels[k].get("fetch_bytes", 0) + kernels[k].get("write_bytes", 0) for k in adj)
     from gpunufft_amd import workloads as W
     w = W.config(WORKLOAD)
@@ -226,7 +227,7 @@ def summarize_trace(path, sha=None, workload="koosh3d_128_mc8"):
              "python3 bench.py --summarize-trace $R/gpurun_out/kt/run_kernel_stats.csv", "```", "",
              "Kernel sources SHA-256 %s (bench.py sources_sha256)." % (sha or sources_sha256()), "",
              "`--profile-steps 3` builds the plan (sector precompute, once) and runs three full "
-             "steps (adjoint: spread, chunk reduction, fold, fused FFT passes z, y, x; forward: "
+             "steps (adjoint: tile spread, tile reduction, fused FFT passes z, y, x; forward: "
              "fused FFT passes x, y, z, interp). `__amd_rocclr_copyBuffer` is the host-to-device "
              "upload of the synthetic workload.", "",
              "| kernel | calls | total us | avg us | % |", "|---|---|---|---|---|"]
@@ -369,8 +370,8 @@ def main():
     achieved = spread_bytes / (spread_ms * 1e-3) / 1e9
     traffic = traffic_summary()
     roofline = {
-        "kernel": "adjoint gridding stage: spread_lane_kernel + reduce_chunks_kernel + "
-                  "fold_kernel (3-D, kernel width 3, 4-coil blocks)",
+        "kernel": "adjoint gridding stage: tile_spread_kernel + tile_reduce_kernel "
+                  "(3-D, kernel width 3, 8-coil groups)",
         "bound": "hbm",
         "achieved": round(achieved, 1),
         "peak": HBM_PEAK_GBS,

@@ -253,15 +253,26 @@ struct gnufft_plan_s {
   Chunk* runs_d = nullptr;
   WorkList work_runs{};
   int lane_per_cu = 0;  // gnufft_plan_set_workgroups_per_cu (0: default)
-  uint32_t* sector_chunks_d = nullptr;  // [S+1] first chunk of each sector
-  uint2* reduce_d = nullptr;            // (first chunk, count) of multi-chunk sectors
-  uint32_t n_reduce = 0;
-  // per-axis padded-sector cover lists of the grid (fold)
-  uint32_t* cover_d = nullptr;
-  Cover cover{};
-  // spread sub-grids, [chunk][padded point][coil], capacity in coils
+  bool cover_ok = true;  // sector_cover_ok
+  // tap table and square roots of the density weights, caller's order
+  float4* taps_d = nullptr;
+  float* dens_sqrt_d = nullptr;
+  // adjoint: the tile lists of the trajectory and the scratch slots of tiles
+  // with several chunks
+  uint32_t* tile_entries_d = nullptr;
+  TileChunk* tile_chunks_d = nullptr;
+  TileTask* tile_tasks_d = nullptr;
+  TileList tiles{};
+  uint32_t n_slots = 0;
+  // partial tiles [slot][coil][tile point], or the fused FFT's intermediate;
+  // capacity in bytes
   float2* scratch_d = nullptr;
-  uint32_t scratch_coils = 0;
+  size_t scratch_cap = 0;
+  // workspace of short trajectories' tables (at most 40 MB) and pinned words
+  // they report through
+  char* short_d = nullptr;
+  size_t short_cap = 0;
+  uint32_t* short_host = nullptr;
   // sensitivities
   float2* sens_d = nullptr;
   uint32_t n_sens = 0;
@@ -302,6 +313,8 @@ void dfree(void* p) {
   if (p) (void)hipFree(p);
 }
 
+size_t round_up_256(size_t b) { return (b + 255) & ~(size_t)255; }
+
 void free_traj(gnufft_plan p) {
   p->generation++;
   p->table_generation++;
@@ -313,19 +326,26 @@ void free_traj(gnufft_plan p) {
   dfree(p->centers_d);
   dfree(p->chunks_d);
   dfree(p->runs_d);
-  dfree(p->sector_chunks_d);
-  dfree(p->reduce_d);
-  dfree(p->scratch_d);
+  dfree(p->taps_d);
+  dfree(p->dens_sqrt_d);
+  dfree(p->tile_entries_d);
+  dfree(p->tile_chunks_d);
+  dfree(p->tile_tasks_d);
   p->traj_sorted_d = p->dens_sorted_d = nullptr;
   p->idx_d = p->assigned_d = p->sdc_d = p->centers_d = nullptr;
   p->chunks_d = nullptr;
   p->runs_d = nullptr;
   p->work_runs = WorkList{};
-  p->sector_chunks_d = nullptr;
-  p->reduce_d = nullptr;
-  p->n_reduce = 0;
-  p->scratch_d = nullptr;
-  p->scratch_coils = 0;
+  p->taps_d = nullptr;
+  p->dens_sqrt_d = nullptr;
+  p->tile_entries_d = nullptr;
+  p->tile_chunks_d = nullptr;
+  p->tile_tasks_d = nullptr;
+  p->tiles.entries = nullptr;
+  p->tiles.chunks = nullptr;
+  p->tiles.tasks = nullptr;
+  p->tiles.n_chunks = p->tiles.n_tasks = 0;
+  p->n_slots = 0;
   p->M = 0;
   p->n_chunks = 0;
   p->work = WorkList{};
@@ -447,41 +467,36 @@ int ensure_grid(gnufft_plan p, uint32_t coils) {
 // Coils processed together: all of them unless the grid would take more
 // than half of the free device memory (coil chunking,
 // CUDA/src/gpuNUFFT_operator.cpp:327-368).
-size_t padded_points(const Geom& g) {
-  return g.dim == 3 ? (size_t)g.P * g.P * g.P : (size_t)g.P * g.P;
-}
-
-// spread sub-grids [chunk][padded point] per coil; the same memory is the
-// fused FFT's intermediate array (used after the fold has consumed it)
-size_t scratch_per_coil(gnufft_plan p) {
-  const size_t sub = (size_t)p->n_chunks * padded_points(p->g);
-  const size_t fft = p->fused_ok ? fused_fft_tmp_elems(p->g) : 0;
+// Scratch of `coils` coils: the spread's partial tiles; the same memory is the
+// fused FFT's intermediate array, used after them.
+size_t scratch_bytes(gnufft_plan p, uint32_t coils) {
+  const size_t sub = (size_t)p->n_slots * tile_points(p->g.dim) * coils;
+  const size_t fft = p->fused_ok ? fused_fft_tmp_elems(p->g) * coils : 0;
   return std::max(sub, fft) * sizeof(float2);
 }
 
-int ensure_scratch(gnufft_plan p, uint32_t coils) {
-  if (p->scratch_coils >= coils) return GNUFFT_OK;
+int ensure_scratch_bytes(gnufft_plan p, size_t bytes) {
+  if (p->scratch_cap >= bytes) return GNUFFT_OK;
   p->generation++;
   dfree(p->scratch_d);
   p->scratch_d = nullptr;
-  p->scratch_coils = 0;
-  const size_t bytes = (size_t)coils * scratch_per_coil(p);
-  if (bytes == 0) return GNUFFT_OK;
+  p->scratch_cap = 0;
   if (hipMalloc(&p->scratch_d, bytes) != hipSuccess)
-    return fail(GNUFFT_ERR_OUT_OF_MEMORY, "spread: sub-grid scratch allocation");
-  p->scratch_coils = coils;
+    return fail(GNUFFT_ERR_OUT_OF_MEMORY, "spread: scratch allocation");
+  p->scratch_cap = bytes;
   return GNUFFT_OK;
 }
 
+int ensure_scratch(gnufft_plan p, uint32_t coils) { return ensure_scratch_bytes(p, scratch_bytes(p, coils)); }
+
 uint32_t coil_batch(gnufft_plan p, uint32_t n_coils) {
   // buffers already hold every coil (steady state, e.g. under graph capture)
-  if (p->grid_coils >= n_coils && p->scratch_coils >= n_coils) return n_coils;
+  if (p->grid_coils >= n_coils && p->scratch_cap >= scratch_bytes(p, n_coils)) return n_coils;
   size_t fr = 0, tot = 0;
   if (hipMemGetInfo(&fr, &tot) != hipSuccess) return 1;
-  // grid + FFT work + spread sub-grids
-  size_t per = (size_t)p->g.Ng * sizeof(float2) * 2 + scratch_per_coil(p);
-  size_t avail = fr / 2 + (size_t)p->grid_coils * p->g.Ng * sizeof(float2) +
-                 (size_t)p->scratch_coils * scratch_per_coil(p);
+  // grid + FFT work + scratch
+  size_t per = (size_t)p->g.Ng * sizeof(float2) * 2 + (scratch_bytes(p, 8) + 7) / 8;
+  size_t avail = fr / 2 + (size_t)p->grid_coils * p->g.Ng * sizeof(float2) + p->scratch_cap;
   size_t cc = per ? avail / per : n_coils;
   if (cc < 1) cc = 1;
   return (uint32_t)std::min<size_t>(cc, n_coils);
@@ -591,73 +606,215 @@ int copy_in(void** dst, const void* src, size_t bytes, int location, hipStream_t
   return GNUFFT_OK;
 }
 
-// Gridding work list from the sector offsets.
-int build_chunks(gnufft_plan p, hipStream_t s) {
-  const uint32_t S = p->S;
-  uint32_t* off_d = nullptr;
-  uint32_t* cnt_d = nullptr;
-  void* temp = nullptr;
-  size_t temp_bytes = 0;
-  HIP_TRY(hipMalloc(&off_d, (S + 1) * sizeof(uint32_t)));
-  p->sector_chunks_d = off_d;  // kept: first chunk of each sector (fold)
-  HIP_TRY(hipMalloc(&cnt_d, (S + 1) * sizeof(uint32_t)));
-  hipError_t e = count_chunks(p->sdc_d, S, p->chunk, cnt_d, off_d, nullptr, &temp_bytes, s);
-  if (e == hipSuccess) e = hipMalloc(&temp, temp_bytes ? temp_bytes : 4);
-  if (e == hipSuccess) e = count_chunks(p->sdc_d, S, p->chunk, cnt_d, off_d, temp, &temp_bytes, s);
-  uint32_t total = 0;
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(&total, off_d + S, sizeof(uint32_t), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  if (e == hipSuccess) e = hipMalloc(&p->chunks_d, (size_t)(total ? total : 1) * sizeof(Chunk));
-  if (e == hipSuccess) e = launch_fill_chunks(p->sdc_d, off_d, S, p->chunk, p->chunks_d, s);
-  std::vector<Chunk> h(total);
-  if (e == hipSuccess && total)
-    e = hipMemcpyAsync(h.data(), p->chunks_d, (size_t)total * sizeof(Chunk), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  dfree(cnt_d);
-  dfree(temp);
-  if (e != hipSuccess) return fail(GNUFFT_ERR_DEVICE, std::string("chunk list: ") + hipGetErrorString(e));
+// Most points per coil that the partial tiles of a plan may take: a million,
+// the FFT's intermediate array or the sector-padded sub-grids of 1024
+// samples, whichever is most.
+double partial_budget(gnufft_plan p) {
+  const Geom& g = p->g;
+  return std::max(std::max(1048576.0, p->fused_ok ? (double)fused_fft_tmp_elems(g) : 0.0),
+                  (double)p->M / 1024.0 * std::pow((double)g.P, g.dim));
+}
+
+// XCD ranges of the plan's `total` sector chunks (sdc: the sectors' offsets)
+// and of their runs; returns the runs, the chunks of each sector merged by up
+// to kInterpRun, unless no sector has several.
+std::vector<Chunk> partition_chunks(gnufft_plan p, const uint32_t* sdc, uint32_t total) {
+  std::vector<uint32_t> counts, run_counts;
+  std::vector<Chunk> runs;
+  counts.reserve(total);
+  for (uint32_t i = 0; i < p->S; i++)
+    for (uint32_t b = sdc[i]; b < sdc[i + 1]; b += p->chunk) counts.push_back(std::min(sdc[i + 1] - b, p->chunk));
   p->n_chunks = total;
-  std::vector<uint32_t> counts(total);
-  for (uint32_t i = 0; i < total; i++) counts[i] = h[i].end - h[i].begin;
   p->work.chunks = p->chunks_d;
   partition_work(counts.data(), total, &p->work);
-  {
-    const uint64_t mean = total ? ((uint64_t)p->M + total - 1) / total : 64;
-    p->round_target = (uint32_t)std::min<uint64_t>(p->chunk, std::max<uint64_t>(64, (mean + 63) / 64 * 64));
-  }
-  // sectors split over several chunks: their sub-grids are summed before the
-  // fold (one workgroup per 256 words of each such sector, so the dense
-  // k-space centre spreads over the whole GPU)
-  std::vector<uint2> tasks;
-  for (uint32_t i = 0; i < total;) {
-    uint32_t j = i + 1;
-    while (j < total && h[j].sector == h[i].sector) j++;
-    if (j - i > 1) tasks.push_back(make_uint2(i, j - i));
-    i = j;
-  }
-  p->n_reduce = (uint32_t)tasks.size();
-  if (!tasks.empty()) {
-    int rc = copy_in((void**)&p->reduce_d, tasks.data(), tasks.size() * sizeof(uint2), GNUFFT_HOST, s);
+  const uint64_t mean = total ? ((uint64_t)p->M + total - 1) / total : 64;
+  p->round_target = (uint32_t)std::min<uint64_t>(p->chunk, std::max<uint64_t>(64, (mean + 63) / 64 * 64));
+  const uint64_t run = (uint64_t)p->chunk * kInterpRun;
+  for (uint32_t i = 0; i < p->S; i++)
+    for (uint64_t b = sdc[i]; b < sdc[i + 1]; b += run) {
+      const uint32_t e = (uint32_t)std::min<uint64_t>(sdc[i + 1], b + run);
+      runs.push_back(Chunk{i, (uint32_t)b, e, 0});
+      run_counts.push_back(e - (uint32_t)b);
+    }
+  if (runs.size() >= total) return {};
+  partition_work(run_counts.data(), (uint32_t)runs.size(), &p->work_runs);
+  return runs;
+}
+
+// Work lists from the sector offsets: the interp's sector chunks, and the
+// tap table and tile lists of the adjoint.
+int build_chunks(gnufft_plan p, hipStream_t s) {
+  const uint32_t S = p->S;
+  const Geom& g = p->g;
+  const uint32_t M = p->M;
+  const uint32_t n_tiles = (uint32_t)p->tiles.nt[0] * p->tiles.nt[1] * p->tiles.nt[2];
+  int key_bits = 1;
+  while ((1ull << key_bits) < n_tiles) key_bits++;
+  uint32_t *off_d = nullptr, *cnt_d = nullptr, *hits_d = nullptr;
+  uint32_t *keys = nullptr, *keys_s = nullptr, *vals = nullptr;
+  uint64_t *hit_off_d = nullptr, *tile_off_d = nullptr;
+  TileTotals* tot_d = nullptr;
+  void *temp = nullptr, *temp2 = nullptr;
+  size_t temp_bytes = 0, need = 0;
+  uint32_t total = 0;
+  uint64_t pairs = 0;
+  TileTotals tot{0, 0, 0};
+  uint32_t chunk = 0;
+  std::vector<uint32_t> sdc((size_t)S + 1);
+  auto run = [&]() -> hipError_t {
+    hipError_t e;
+#define STEP(x) \
+  if ((e = (x)) != hipSuccess) return e
+    STEP(hipMalloc(&off_d, (S + 1) * sizeof(uint32_t)));
+    STEP(hipMalloc(&cnt_d, (S + 1) * sizeof(uint32_t)));
+    STEP(hipMalloc(&hits_d, (size_t)std::max(M, 1u) * sizeof(uint32_t)));
+    STEP(hipMalloc(&hit_off_d, ((size_t)M + 1) * sizeof(uint64_t)));
+    STEP(hipMalloc(&p->taps_d, (size_t)std::max(M, 1u) * g.dim * tap_vec(g.kw) * sizeof(float4)));
+    if (p->dens_sorted_d) STEP(hipMalloc(&p->dens_sqrt_d, (size_t)std::max(M, 1u) * sizeof(float)));
+    STEP(hipMalloc(&tile_off_d, ((size_t)n_tiles + 1) * sizeof(uint64_t)));
+    STEP(hipMalloc(&tot_d, ((size_t)n_tiles + 1) * sizeof(TileTotals)));
+    STEP(count_chunks(p->sdc_d, S, p->chunk, cnt_d, off_d, nullptr, &temp_bytes, s));
+    STEP(scan_counts(nullptr, &need, hits_d, hit_off_d, M, s));
+    temp_bytes = std::max(temp_bytes, need);
+    STEP(scan_tile_chunks(nullptr, &need, tile_off_d, n_tiles, 1, tot_d, s));
+    temp_bytes = std::max(temp_bytes, need);
+    STEP(hipMalloc(&temp, temp_bytes ? temp_bytes : 4));
+    STEP(count_chunks(p->sdc_d, S, p->chunk, cnt_d, off_d, temp, &temp_bytes, s));
+    STEP(launch_taps(g, p->traj_sorted_d, p->dens_sorted_d, p->idx_d, p->lut_d, p->taps_d, p->dens_sqrt_d, hits_d, s));
+    STEP(scan_counts(temp, &temp_bytes, hits_d, hit_off_d, M, s));
+    STEP(hipMemcpyAsync(&total, off_d + S, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    STEP(hipMemcpyAsync(&pairs, hit_off_d + M, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+    STEP(hipStreamSynchronize(s));
+    const size_t room = (size_t)(pairs ? pairs : 1);
+    STEP(hipMalloc(&p->chunks_d, (size_t)(total ? total : 1) * sizeof(Chunk)));
+    STEP(launch_fill_chunks(p->sdc_d, off_d, S, p->chunk, p->chunks_d, s));
+    STEP(hipMemcpyAsync(sdc.data(), p->sdc_d, sdc.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    STEP(hipMalloc(&keys, room * sizeof(uint32_t)));
+    STEP(hipMalloc(&keys_s, room * sizeof(uint32_t)));
+    STEP(hipMalloc(&vals, room * sizeof(uint32_t)));
+    STEP(hipMalloc(&p->tile_entries_d, room * sizeof(uint32_t)));
+    STEP(launch_emit_pairs(g, p->tiles, p->taps_d, hit_off_d, keys, vals, s));
+    if (pairs) {
+      STEP(sort_tile_pairs(nullptr, &need, keys, keys_s, vals, p->tile_entries_d, pairs, key_bits, s));
+      STEP(hipMalloc(&temp2, need ? need : 4));
+      STEP(sort_tile_pairs(temp2, &need, keys, keys_s, vals, p->tile_entries_d, pairs, key_bits, s));
+    }
+    STEP(launch_tile_offsets(keys_s, pairs, n_tiles, tile_off_d, s));
+    // larger chunks when the partial tiles would not stay within their budget
+    for (chunk = tile_chunk(g.dim, pairs);; chunk *= 2) {
+      STEP(scan_tile_chunks(temp, &temp_bytes, tile_off_d, n_tiles, chunk, tot_d, s));
+      STEP(hipMemcpyAsync(&tot, tot_d + n_tiles, sizeof(TileTotals), hipMemcpyDeviceToHost, s));
+      STEP(hipStreamSynchronize(s));
+      if ((double)tot.slots * tile_points(g.dim) <= partial_budget(p) || chunk >= (1u << 30)) break;
+    }
+    STEP(hipMalloc(&p->tile_chunks_d, (size_t)tot.chunks * sizeof(TileChunk)));
+    STEP(hipMalloc(&p->tile_tasks_d, (size_t)(tot.tasks ? tot.tasks : 1) * sizeof(TileTask)));
+    STEP(fill_tile_chunks(tile_off_d, n_tiles, chunk, tot_d, p->tile_chunks_d, p->tile_tasks_d, s));
+#undef STEP
+    return hipStreamSynchronize(s);
+  };
+  const hipError_t e = run();
+  if (e != hipSuccess) (void)hipStreamSynchronize(s);  // copies into locals
+  for (void* q : {(void*)off_d, (void*)cnt_d, (void*)hits_d, (void*)hit_off_d, (void*)keys, (void*)keys_s,
+                  (void*)vals, (void*)tot_d, (void*)tile_off_d, temp, temp2})
+    dfree(q);
+  if (e != hipSuccess) return fail(GNUFFT_ERR_DEVICE, std::string("chunk list: ") + hipGetErrorString(e));
+  p->tiles.entries = p->tile_entries_d;
+  p->tiles.chunks = p->tile_chunks_d;
+  p->tiles.tasks = p->tile_tasks_d;
+  p->tiles.n_chunks = tot.chunks;
+  p->tiles.n_tasks = tot.tasks;
+  p->n_slots = tot.slots;
+  const std::vector<Chunk> runs = partition_chunks(p, sdc.data(), total);
+  if (!runs.empty()) {
+    int rc = copy_in((void**)&p->runs_d, runs.data(), runs.size() * sizeof(Chunk), GNUFFT_HOST, s);
     if (rc) return rc;
-    std::vector<Chunk> runs;
-    std::vector<uint32_t> run_counts;
-    for (uint32_t i = 0; i < total;) {
-      uint32_t j = i + 1;
-      while (j < total && j - i < (uint32_t)kInterpRun && h[j].sector == h[i].sector) j++;
-      runs.push_back(Chunk{h[i].sector, h[i].begin, h[j - 1].end, 0});
-      run_counts.push_back(h[j - 1].end - h[i].begin);
-      i = j;
-    }
-    rc = copy_in((void**)&p->runs_d, runs.data(), runs.size() * sizeof(Chunk), GNUFFT_HOST, s);
-    if (rc) {
-      (void)hipStreamSynchronize(s);  // the task upload above reads `tasks`
-      return rc;
-    }
     p->work_runs.chunks = p->runs_d;
-    partition_work(run_counts.data(), (uint32_t)runs.size(), &p->work_runs);
     HIP_TRY(hipStreamSynchronize(s));
   }
+  return GNUFFT_OK;
+}
+
+// build_chunks and the sector tables of a short trajectory, M > 0 samples in
+// device or host memory.
+int build_short(gnufft_plan p, const float* traj, uint32_t M, const float* dens, int location, hipStream_t s) {
+  const Geom& g = p->g;
+  const uint32_t S = p->S, D = (uint32_t)g.dim;
+  ShortTables t{};
+  t.lut = p->lut_d;
+  t.S = S;
+  t.n_tiles = (uint32_t)p->tiles.nt[0] * p->tiles.nt[1] * p->tiles.nt[2];
+  t.chunk = p->chunk;
+  const size_t words = short_tables_words(M, S, t.n_tiles), entries = short_tables_entries(g, M);
+  size_t temp_bytes = 0;
+  p->M = M;
+  p->g.M = (int)M;
+  t.max_slots = (uint32_t)std::min(partial_budget(p) / tile_points(g.dim), 4e9);
+  auto run = [&]() -> hipError_t {
+    hipError_t e;
+#define STEP(x) \
+  if ((e = (x)) != hipSuccess) return e
+    STEP(launch_short_tables(g, p->tiles, t, nullptr, &temp_bytes, s));
+    // the workspace: input, counts, offsets, the scan's temporary
+    const size_t in_b = round_up_256(((size_t)D + 1) * M * 4), words_b = round_up_256(words * 4);
+    const size_t need = in_b + 2 * words_b + temp_bytes;
+    if (p->short_cap < need) {
+      dfree(p->short_d);
+      p->short_d = nullptr;
+      p->short_cap = 0;
+      STEP(hipMalloc((void**)&p->short_d, need));
+      p->short_cap = need;
+    }
+    if (!p->short_host)
+      STEP(hipHostMalloc((void**)&p->short_host, ((size_t)S + 1 + kShortTotals) * 4, hipHostMallocDefault));
+    float* in = reinterpret_cast<float*>(p->short_d);
+    const hipMemcpyKind kind = location == GNUFFT_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
+    STEP(hipMemcpyAsync(in, traj, (size_t)D * M * 4, kind, s));
+    t.traj = in;
+    if (dens) {
+      STEP(hipMemcpyAsync(in + (size_t)D * M, dens, (size_t)M * 4, kind, s));
+      t.dens = in + (size_t)D * M;
+      STEP(hipMalloc(&p->dens_sorted_d, (size_t)M * 4));
+      STEP(hipMalloc(&p->dens_sqrt_d, (size_t)M * 4));
+    }
+    t.counts = reinterpret_cast<uint32_t*>(p->short_d + in_b);
+    t.offs = reinterpret_cast<uint32_t*>(p->short_d + in_b + words_b);
+    const size_t n_chunks = (size_t)S + M / t.chunk, n_tile_chunks = t.n_tiles + entries / 128;
+    STEP(hipMalloc(&p->assigned_d, (size_t)M * 4));
+    STEP(hipMalloc(&p->idx_d, (size_t)M * 4));
+    STEP(hipMalloc(&p->traj_sorted_d, (size_t)M * D * 4));
+    STEP(hipMalloc(&p->sdc_d, ((size_t)S + 1) * 4));
+    STEP(hipMalloc(&p->centers_d, (size_t)S * D * 4));
+    STEP(hipMalloc(&p->chunks_d, n_chunks * sizeof(Chunk)));
+    STEP(hipMalloc(&p->runs_d, n_chunks * sizeof(Chunk)));
+    STEP(hipMalloc(&p->taps_d, (size_t)M * D * tap_vec(g.kw) * sizeof(float4)));
+    STEP(hipMalloc(&p->tile_entries_d, entries * sizeof(uint32_t)));
+    STEP(hipMalloc(&p->tile_chunks_d, n_tile_chunks * sizeof(TileChunk)));
+    STEP(hipMalloc(&p->tile_tasks_d, t.n_tiles * sizeof(TileTask)));
+    t.assigned = p->assigned_d, t.idx = p->idx_d, t.sdc = p->sdc_d, t.centers = p->centers_d;
+    t.traj_sorted = p->traj_sorted_d, t.dens_sorted = p->dens_sorted_d;
+    t.chunks = p->chunks_d, t.runs = p->runs_d;
+    t.taps = p->taps_d, t.dens_sqrt = p->dens_sqrt_d, t.entries = p->tile_entries_d;
+    t.tile_chunks = p->tile_chunks_d, t.tile_tasks = p->tile_tasks_d;
+    t.host = p->short_host;
+    STEP(launch_short_tables(g, p->tiles, t, p->short_d + in_b + 2 * words_b, &temp_bytes, s));
+#undef STEP
+    return hipSuccess;
+  };
+  hipError_t e = run();
+  const hipError_t waited = hipStreamSynchronize(s);
+  if (e == hipSuccess) e = waited;
+  if (e != hipSuccess)
+    return fail(e == hipErrorOutOfMemory ? GNUFFT_ERR_OUT_OF_MEMORY : GNUFFT_ERR_DEVICE,
+                std::string("set_trajectory: ") + hipGetErrorString(e));
+  const uint32_t* totals = p->short_host + S + 1;
+  p->tiles.entries = p->tile_entries_d;
+  p->tiles.chunks = p->tile_chunks_d;
+  p->tiles.tasks = p->tile_tasks_d;
+  p->tiles.n_chunks = totals[2];
+  p->n_slots = totals[3];
+  p->tiles.n_tasks = totals[4];
+  if (!partition_chunks(p, p->short_host, totals[0]).empty()) p->work_runs.chunks = p->runs_d;
   return GNUFFT_OK;
 }
 
@@ -669,20 +826,21 @@ SpreadArgs spread_args(gnufft_plan p, const float2* data, float2* grid, uint32_t
   SpreadArgs a{};
   a.data = data;
   a.coil_stride = p->M;
-  a.crds = p->traj_sorted_d;
-  a.work = p->work;
-  a.lut = p->lut_d;
+  a.taps = p->taps_d;
+  a.tiles = p->tiles;
   a.scratch = p->scratch_d;
-  a.sector_chunks = p->sector_chunks_d;
-  a.reduce_tasks = p->reduce_d;
-  a.n_reduce = p->n_reduce;
-  a.cover = p->cover;
   a.grid = grid;
   a.n_coils = (int)n_coils;
-  a.lane_per_cu = p->lane_per_cu;
   return a;
 }
 
+// Spread of a plan; geometries whose padded sectors do not fit the device
+// are refused.
+hipError_t plan_spread(gnufft_plan p, const SpreadArgs& a, hipStream_t s) {
+  if (a.n_coils == 0) return hipSuccess;
+  if (!p->cover_ok || (p->n_chunks > 0 && !spread_supported(p->g))) return hipErrorInvalidValue;
+  return launch_spread(p->g, a, s);
+}
 
 }  // namespace
 
@@ -833,17 +991,10 @@ int gnufft_plan_create(gnufft_plan* plan, const uint32_t img_dims[3], uint32_t k
     p->fused = p->fused_ok && fused_fft_preferred(g);
   }
   if (rc == GNUFFT_OK) {
-    std::vector<uint32_t> words;
-    size_t base[6];
-    build_cover(g, &words, base, p->cover.max_len, &p->cover.max_cov);
-    rc = copy_in((void**)&p->cover_d, words.data(), words.size() * sizeof(uint32_t), GNUFFT_HOST, s);
-    if (rc == GNUFFT_OK) {
-      for (int a = 0; a < 3; a++) {
-        p->cover.off[a] = p->cover_d + base[a];
-        p->cover.ent[a] = p->cover_d + base[3 + a];
-      }
-      if (hipStreamSynchronize(s) != hipSuccess) rc = fail(GNUFFT_ERR_DEVICE, "plan_create: cover lists");
-    }
+    for (int a = 0; a < 3; a++)
+      p->tiles.nt[a] = a < g.dim ? (g.G[a] + 4 * tile_width(g.dim, a) - 1) / (4 * tile_width(g.dim, a)) * 4 : 1;
+    p->cover_ok = sector_cover_ok(g);
+    if (hipStreamSynchronize(s) != hipSuccess) rc = fail(GNUFFT_ERR_DEVICE, "plan_create: tables");
   }
   if (rc != GNUFFT_OK) {
     gnufft_plan_destroy(p);
@@ -909,9 +1060,11 @@ int gnufft_plan_destroy(gnufft_plan p) {
   p->timer.collect();
   free_traj(p);
   free_ffts(p);
+  dfree(p->scratch_d);
+  dfree(p->short_d);
+  if (p->short_host) (void)hipHostFree(p->short_host);
   dfree(p->lut_d);
   dfree(p->deapo_d);
-  dfree(p->cover_d);
   dfree(p->sens_d);
   dfree(p->grid_d);
   dfree(p->img_tmp_d);
@@ -955,6 +1108,11 @@ int gnufft_plan_set_trajectory(gnufft_plan p, const float* traj, uint32_t n_samp
   free_traj(p);
   const uint32_t M = n_samples;
   const int D = p->g.dim;
+  if (short_tables_ok(M, p->S, (uint32_t)p->tiles.nt[0] * p->tiles.nt[1] * p->tiles.nt[2])) {
+    const int rc = build_short(p, traj, M, dens, location, s);
+    if (rc != GNUFFT_OK) free_traj(p);
+    return rc;
+  }
   float* traj_in = nullptr;
   float* dens_in = nullptr;
   uint32_t *keys = nullptr, *vals = nullptr, *keys_sorted = nullptr;
@@ -1225,14 +1383,17 @@ int gnufft_spread_sorted(gnufft_plan p, const void* data_sorted, void* grid, uin
   if (!p->sdc_d) return fail(GNUFFT_ERR_STATE, "spread_sorted: no trajectory set");
   hipStream_t s = (hipStream_t)stream;
   const uint32_t cc = coil_batch(p, n_coils);
-  int rc = ensure_scratch(p, cc);
+  // partial tiles and the samples brought to the caller's order
+  const size_t part = (size_t)p->n_slots * tile_points(p->g.dim) * cc;
+  int rc = ensure_scratch_bytes(p, (part + (size_t)p->M * cc) * sizeof(float2));
   if (rc) return rc;
   for (uint32_t c0 = 0; c0 < n_coils; c0 += cc) {
     const uint32_t nc = std::min(cc, n_coils - c0);
-    SpreadArgs a = spread_args(p, (const float2*)data_sorted + (size_t)c0 * p->M,
-                               (float2*)grid + (size_t)c0 * p->g.Ng, nc);
+    float2* data = p->scratch_d + part;
+    HIP_TRY(launch_unsort((const float2*)data_sorted + (size_t)c0 * p->M, p->M, p->M, (int)nc, p->idx_d, data, s));
+    SpreadArgs a = spread_args(p, data, (float2*)grid + (size_t)c0 * p->g.Ng, nc);
     a.fold_shift = false;
-    TIMED(p, GNUFFT_T_SPREAD, s, launch_spread(p->g, a, (int)p->round_target, s));
+    TIMED(p, GNUFFT_T_SPREAD, s, plan_spread(p, a, s));
   }
   return GNUFFT_OK;
 }
@@ -1282,10 +1443,9 @@ int gnufft_adjoint(gnufft_plan p, const void* kdata, void* out, uint32_t n_coils
     float2* grid = grid_out ? (float2*)out + (size_t)c0 * g.Ng : p->grid_d;
     {
       SpreadArgs a = spread_args(p, (const float2*)kdata + (size_t)c0 * p->M, grid, nc);
-      a.gather = p->idx_d;
-      a.dens = p->dens_sorted_d;
+      a.dens = p->dens_sqrt_d;
       a.fold_shift = !grid_out;
-      TIMED(p, GNUFFT_T_SPREAD, s, launch_spread(g, a, (int)p->round_target, s));
+      TIMED(p, GNUFFT_T_SPREAD, s, plan_spread(p, a, s));
     }
     if (grid_out) continue;
     if (p->fused) {
@@ -1395,6 +1555,8 @@ int gnufft_forward(gnufft_plan p, const void* img, void* out, uint32_t n_coils, 
 // ---------------------------------------------------------------------------
 }  // extern "C"
 
+constexpr int kSpreadNc[3] = {2, 4, 8};  // coil-group sizes of the batched spread
+
 struct gnufft_batch_s {
   int dim = 2, nx = 4;
   std::vector<gnufft_plan> plans;  // in batch order (grouped by grid size)
@@ -1404,14 +1566,10 @@ struct gnufft_batch_s {
   std::vector<BatchOp> ops_h;
   BatchOp* ops_d = nullptr;
   uint4* items_d = nullptr;
-  BatchList spread{}, interp{}, fold{}, reduce{}, post{}, pre{};
-  // lane kernels: chunks of at most 2 * kBatchSmallThreads samples, run in
-  // small workgroups (spread and interp share the lists)
-  BatchList spread_small{}, interp_small{};
-  size_t spread_lds = 0, interp_lds = 0, spread_small_lds = 0, interp_small_lds = 0;
-  int fold_threads = 64;
-  bool fold_generic = false;  // some plan needs the fold's generic body
-  uint32_t max_kstride = 0;
+  // spread: one list per coil-group size (kSpreadNc); interp, lane kernels:
+  // chunks of at most 2 * kBatchSmallThreads samples run in small workgroups
+  BatchList spread[3]{}, reduce{}, interp{}, interp_small{}, post{}, pre{};
+  size_t spread_lds[3] = {0, 0, 0}, interp_lds = 0, interp_small_lds = 0;
   float2* grid_d = nullptr;
   float2* scratch_d = nullptr;
   struct Group {
@@ -1570,8 +1728,8 @@ int gnufft_batch_create(gnufft_batch* batch, const gnufft_plan* plans, uint32_t 
     grid_off[k] = grid_total;
     grid_total += (size_t)C * p->g.Ng;
     scratch_off[k] = scratch_total;
-    // spread sub-grids, then (fused FFT) the transform's intermediate array
-    scratch_total += std::max((size_t)p->n_chunks * C * padded_points(p->g),
+    // partial tiles, then (fused FFT) the transform's intermediate array
+    scratch_total += std::max((size_t)p->n_slots * C * tile_points(p->g.dim),
                               batch_fused(p) ? (size_t)C * fused_fft_tmp_elems(p->g) : (size_t)0);
     // rocFFT groups: runs of consecutive non-fused plans of one grid size
     if (!batch_fused(p)) {
@@ -1589,22 +1747,20 @@ int gnufft_batch_create(gnufft_batch* batch, const gnufft_plan* plans, uint32_t 
     return fail(GNUFFT_ERR_OUT_OF_MEMORY, "batch_create: grid / scratch allocation");
   }
   // descriptors and item lists
-  // (chunk, coil block) items of large (sp) and small (ss) chunks
-  std::vector<uint4> sp, ss, rd, fo, po, pr;
-  std::vector<uint32_t> sp_cost, ss_cost, fo_cost;
+  // spread items (tile chunk, coil group) by group size; interp items (chunk,
+  // coil block) of large (il) and small (is) chunks
+  std::vector<uint4> sp[3], il, is, rd, po, pr;
+  std::vector<uint32_t> sp_cost[3], il_cost, is_cost;
   for (uint32_t k = 0; k < n_plans && !rc; k++) {
     const gnufft_plan p = b->plans[k];
     const uint32_t C = b->coils[k];
-    const uint32_t cbs = (C + grid_cb - 1) / grid_cb;  // spread / interp coil blocks
+    const uint32_t cbs = (C + grid_cb - 1) / grid_cb;  // interp coil blocks
     BatchOp op{};
     op.g = p->g;
     op.s = spread_args(p, nullptr, b->grid_d + grid_off[k], C);
     op.s.scratch = b->scratch_d + scratch_off[k];
-    op.s.gather = p->idx_d;
-    op.s.dens = p->dens_sorted_d;
+    op.s.dens = p->dens_sqrt_d;
     op.s.fold_shift = true;
-    op.s.n_reduce = 0;
-    op.s.sub_cb = lane ? kBatchLaneCB : kBatchCB;  // the batched spread's coil block
     op.i.grid = b->grid_d + grid_off[k];
     op.i.crds = p->traj_sorted_d;
     op.i.work = p->work;
@@ -1619,29 +1775,21 @@ int gnufft_batch_create(gnufft_batch* batch, const gnufft_plan* plans, uint32_t 
                        p->n_sens ? p->sens_d : nullptr, nullptr, GNUFFT_STOP_DEAPODIZATION};
     op.pre = PreArgs{nullptr, p->n_sens ? 0 : 1, p->n_sens ? p->sens_d : nullptr, p->deapo_d,
                      b->grid_d + grid_off[k], (int)C};
-    op.R_spread = batch_round(spread_round, p->g, (int)p->round_target, 0);
     op.R_interp = batch_round(interp_round, p->g, (int)p->round_target, 3072);
-    if (op.R_spread <= 0 || op.R_interp <= 0) {
+    if (!padded_sector_fits(p->g, kBatchCB) || op.R_interp <= 0) {
       rc = fail(GNUFFT_ERR_UNSUPPORTED, "batch_create: padded sector does not fit in LDS");
       break;
     }
     if (lane) {
-      b->spread_lds = std::max(b->spread_lds, lane_lds_bytes(p->g, kBatchLaneCB));
-      b->spread_small_lds = std::max(b->spread_small_lds, lane_lds_bytes(p->g, kBatchLaneCB, false));
-      b->interp_small_lds = b->spread_small_lds;
+      b->interp_small_lds = std::max(b->interp_small_lds, lane_lds_bytes(p->g, kBatchLaneCB, false));
       b->interp_lds = std::max(b->interp_lds, lane_lds_bytes(p->g, kBatchLaneCB));
     } else {
-      b->spread_lds = std::max(b->spread_lds, spread_lds_bytes(p->g, kBatchCB, op.R_spread));
       b->interp_lds = std::max(b->interp_lds, interp_lds_bytes(p->g, kBatchCB, op.R_interp));
     }
-    const int ft = fold_threads(p->g, p->cover);
-    if (ft == 0) {
-      rc = fail(GNUFFT_ERR_UNSUPPORTED, "batch_create: too many fold candidates");
+    if (!p->cover_ok) {
+      rc = fail(GNUFFT_ERR_UNSUPPORTED, "batch_create: too many sectors cover a point");
       break;
     }
-    b->fold_threads = std::max(b->fold_threads, ft);
-    b->fold_generic = b->fold_generic || fold_generic(p->cover);
-    b->max_kstride = std::max<uint32_t>(b->max_kstride, C * (uint32_t)padded_points(p->g));
     b->ops_h.push_back(op);
     if (b->fused) b->fft_desc_h.resize((k + 1) * fused_fft_desc_bytes());
     if (batch_fused(p)) {
@@ -1653,10 +1801,12 @@ int gnufft_batch_create(gnufft_batch* batch, const gnufft_plan* plans, uint32_t 
         break;
       }
     }
-    // chunk list (host copy) for the gridding items and the reduce tasks
+    // chunk lists (host copies) for the gridding items and the reduce tasks
     std::vector<Chunk> ch(p->n_chunks);
-    if (p->n_chunks &&
-        hipMemcpy(ch.data(), p->chunks_d, ch.size() * sizeof(Chunk), hipMemcpyDeviceToHost) != hipSuccess) {
+    std::vector<TileChunk> tc(p->tiles.n_chunks);
+    if ((p->n_chunks &&
+         hipMemcpy(ch.data(), p->chunks_d, ch.size() * sizeof(Chunk), hipMemcpyDeviceToHost) != hipSuccess) ||
+        hipMemcpy(tc.data(), p->tile_chunks_d, tc.size() * sizeof(TileChunk), hipMemcpyDeviceToHost) != hipSuccess) {
       rc = fail(GNUFFT_ERR_DEVICE, "batch_create: chunk list copy");
       break;
     }
@@ -1664,22 +1814,22 @@ int gnufft_batch_create(gnufft_batch* batch, const gnufft_plan* plans, uint32_t 
       const uint32_t n = ch[ci].end - ch[ci].begin;
       const bool small = lane && n <= 2u * (uint32_t)kBatchSmallThreads;
       for (uint32_t cb = 0; cb < cbs; cb++) {
-        (small ? ss : sp).push_back(make_uint4(k, ci, cb, 0));
-        (small ? ss_cost : sp_cost).push_back(n + (small ? 100u : 300u));
+        (small ? is : il).push_back(make_uint4(k, ci, cb, 0));
+        (small ? is_cost : il_cost).push_back(n + (small ? 100u : 300u));
       }
     }
-    for (uint32_t i = 0; i < p->n_chunks;) {
-      uint32_t j = i + 1;
-      while (j < p->n_chunks && ch[j].sector == ch[i].sector) j++;
-      if (j - i > 1) rd.push_back(make_uint4(k, i, j - i, 0));
-      i = j;
-    }
-    const uint32_t fcbs = (C + kBatchCB - 1) / kBatchCB;  // fold coil blocks
-    for (uint32_t sct = 0; sct < p->S; sct++)
-      for (uint32_t cb = 0; cb < fcbs; cb++) {
-        fo.push_back(make_uint4(k, sct, cb, 0));
-        fo_cost.push_back(1u);
+    int q = 0;
+    while (kSpreadNc[q] < tile_coils((int)C)) q++;
+    b->spread_lds[q] = spread_lds_bytes(p->g.dim, kSpreadNc[q]);
+    for (uint32_t ci = 0; ci < p->tiles.n_chunks; ci++)
+      for (uint32_t cg = 0; cg * kSpreadNc[q] < C; cg++) {
+        sp[q].push_back(make_uint4(k, ci, cg, 0));
+        sp_cost[q].push_back(tc[ci].n + 100u);
       }
+    for (uint32_t t = 0; t < p->tiles.n_tasks; t++)
+      for (uint32_t c = 0; c < C; c++)
+        for (int blk = 0; blk < tile_points(p->g.dim) / 256; blk++)
+          rd.push_back(make_uint4(k, t, c, (uint32_t)blk));
     if (!batch_fused(p)) {  // pre / post run beside rocFFT; the fused FFT has them inside
       for (uint64_t blk = 0; blk * 256 < (uint64_t)p->g.Ni; blk++) po.push_back(make_uint4(k, (uint32_t)blk, 0, 0));
       for (uint64_t blk = 0; blk * 256 < (uint64_t)p->g.Ng; blk++) pr.push_back(make_uint4(k, (uint32_t)blk, 0, 0));
@@ -1687,10 +1837,10 @@ int gnufft_batch_create(gnufft_batch* batch, const gnufft_plan* plans, uint32_t 
   }
   if (!rc) {
     std::vector<uint4> all;
-    all.insert(all.end(), sp.begin(), sp.end());
-    all.insert(all.end(), ss.begin(), ss.end());
+    for (auto& v : sp) all.insert(all.end(), v.begin(), v.end());
+    all.insert(all.end(), il.begin(), il.end());
+    all.insert(all.end(), is.begin(), is.end());
     all.insert(all.end(), rd.begin(), rd.end());
-    all.insert(all.end(), fo.begin(), fo.end());
     all.insert(all.end(), po.begin(), po.end());
     all.insert(all.end(), pr.begin(), pr.end());
     if (hipMalloc(&b->ops_d, b->ops_h.size() * sizeof(BatchOp)) != hipSuccess ||
@@ -1712,12 +1862,10 @@ int gnufft_batch_create(gnufft_batch* batch, const gnufft_plan* plans, uint32_t 
       }
       at += v.size();
     };
-    list(b->spread, sp, &sp_cost);
-    b->interp = b->spread;
-    list(b->spread_small, ss, &ss_cost);
-    b->interp_small = b->spread_small;
+    for (int q = 0; q < 3; q++) list(b->spread[q], sp[q], &sp_cost[q]);
+    list(b->interp, il, &il_cost);
+    list(b->interp_small, is, &is_cost);
     list(b->reduce, rd, nullptr);
-    list(b->fold, fo, &fo_cost);
     list(b->post, po, nullptr);
     list(b->pre, pr, nullptr);
     if (b->fused) {
@@ -1798,10 +1946,9 @@ int gnufft_batch_adjoint(gnufft_batch b, const void* const* kdata, void* const* 
   }
   int rc = batch_upload_ops(b, s);
   if (rc) return rc;
-  HIP_TRY(launch_spread_batch(b->dim, b->nx, b->ops_d, b->spread, b->spread_lds, s));
-  HIP_TRY(launch_spread_batch_small(b->dim, b->ops_d, b->spread_small, b->spread_small_lds, s));
-  HIP_TRY(launch_reduce_batch(b->ops_d, b->reduce, b->max_kstride, s));
-  HIP_TRY(launch_fold_batch(b->dim, b->ops_d, b->fold, b->fold_threads, b->fold_generic, s));
+  for (int q = 0; q < 3; q++)
+    HIP_TRY(launch_spread_batch(b->dim, b->nx == 8 ? 8 : 4, kSpreadNc[q], b->ops_d, b->spread[q], b->spread_lds[q], s));
+  HIP_TRY(launch_tile_reduce_batch(b->dim, b->ops_d, b->reduce, s));
   if (b->fused) {
     for (int ps = 0; ps < fused_fft_pass_count(b->dim); ps++) {
       HIP_TRY(launch_fused_fft_batch(b->dim, true, ps, false, b->fft_prime, b->fft_desc_d,
@@ -1894,7 +2041,6 @@ int noalloc_area(unsigned char** out) {
   return GNUFFT_OK;
 }
 
-size_t round_up_256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 }  // namespace
 
@@ -1919,7 +2065,7 @@ int gnufft_adjoint_noalloc(gnufft_plan p, const void* kdata, void* out, uint32_t
   // per coil: work grid (unless the caller's buffer is the grid) and the
   // spread sub-grids / fused FFT intermediate
   const size_t grid_b = grid_out ? 0 : (size_t)g.Ng * sizeof(float2);
-  const size_t scr_b = scratch_per_coil(p);
+  const size_t scr_b = scratch_bytes(p, 1);
   const size_t per = round_up_256(grid_b) + round_up_256(scr_b);
   if (per == 0 || per > kNoAllocBytes)
     return fail(GNUFFT_ERR_UNSUPPORTED,
@@ -1938,10 +2084,9 @@ int gnufft_adjoint_noalloc(gnufft_plan p, const void* kdata, void* out, uint32_t
     float2* scr = (float2*)(area + round_up_256(grid_b * nc));
     SpreadArgs a = spread_args(p, (const float2*)kdata + (size_t)c0 * p->M, grid, nc);
     a.scratch = scr;
-    a.gather = p->idx_d;
-    a.dens = p->dens_sorted_d;
+    a.dens = p->dens_sqrt_d;
     a.fold_shift = !grid_out;
-    HIP_TRY(launch_spread(g, a, (int)p->round_target, s));
+    HIP_TRY(plan_spread(p, a, s));
     if (grid_out) continue;
     float2* dst = use_sens ? (float2*)out : (float2*)out + (size_t)c0 * g.Ni;
     HIP_TRY(fused_fft_adjoint(g, grid, scr, (int)nc, p->deapo_d,

@@ -57,6 +57,95 @@ struct Chunk {
 };
 
 // ---------------------------------------------------------------------------
+// Tap table: per axis and sample (caller's order) the first grid index of the
+// sample's taps, in [0, G), and its kw weights (zero where the reference skips a tap;
+// the (kw + 1)-th tap of a position exactly half-way between grid points is
+// at the kernel's edge and has weight zero). tap_vec(kw) float4 per entry:
+// word 0 the index (as an int), then the weights, zeros past the last.
+// ---------------------------------------------------------------------------
+__host__ __device__ constexpr int tap_vec(int kw) { return kw <= 3 ? 1 : 2; }
+
+// ---------------------------------------------------------------------------
+// Tiles of the adjoint gridding (spread.hip): the grid cut into tiles of
+// tile_width(dim, axis) points, each with the list of the samples that have a
+// tap of nonzero weight inside it. Sixteen points in x are whole 128-byte
+// lines of the grid. A tile is worked on as sub-tiles of 4 points in x (3-D:
+// by 4 in y).
+// ---------------------------------------------------------------------------
+__host__ __device__ constexpr int tile_width(int dim, int axis) {
+  return axis == 0 ? 16 : axis == 1 ? (dim == 3 ? 8 : 16) : (dim == 3 ? 4 : 1);
+}
+__host__ __device__ constexpr int tile_points(int dim) {
+  return tile_width(dim, 0) * tile_width(dim, 1) * tile_width(dim, 2);
+}
+__host__ __device__ constexpr int tile_subs(int dim) { return dim == 3 ? 8 : 4; }
+// Coils per workgroup of the spread: the block's 16 columns are 8 / NC
+// points in x times NC coils.
+__host__ __device__ constexpr int tile_coils(int n_coils) {
+  return n_coils > 4 ? 8 : n_coils > 2 ? 4 : 2;
+}
+constexpr uint32_t kNoSlot = ~0u;
+
+struct TileChunk {  // list entries [begin, begin + n) of a tile
+  uint64_t begin;
+  uint32_t n;  // 0: an empty tile
+  uint32_t tile;
+  uint32_t slot;  // scratch slot of a tile with several chunks, else kNoSlot
+  uint32_t pad;
+};
+
+struct TileTask {  // a tile with several chunks: slots [slot, slot + count)
+  uint32_t tile, slot, count, pad;
+};
+
+struct TileList {
+  const uint32_t* entries;  // sample numbers, caller's order
+  const TileChunk* chunks;  // every tile has at least one (an empty tile is cleared)
+  const TileTask* tasks;
+  uint32_t n_chunks, n_tasks;
+  int nt[3];  // tiles per axis, rounded up to a multiple of 4 (1 on an unused axis)
+};
+
+struct TileTotals {
+  uint32_t chunks, slots, tasks;
+};
+
+#if defined(__HIPCC__)
+// First point of a tile. Tiles are numbered in blocks of 4 per axis (nt is a
+// multiple of 4 on the axes in use), so that neighbouring numbers are
+// neighbours on every axis; tiles past the grid's end are empty.
+template <int DIM>
+__device__ inline void tile_start(const TileList& l, uint32_t tile, int* t0) {
+  constexpr uint32_t per = DIM == 3 ? 64 : 16;
+  const uint32_t in = tile % per, b = tile / per;
+  const uint32_t bx = (uint32_t)l.nt[0] / 4, by = (uint32_t)l.nt[1] / 4;
+  t0[0] = (int)((b % bx) * 4 + (in & 3)) * tile_width(DIM, 0);
+  t0[1] = (int)((DIM == 3 ? (b / bx) % by : b / bx) * 4 + ((in >> 2) & 3)) * tile_width(DIM, 1);
+  t0[2] = DIM == 3 ? (int)((b / (bx * by)) * 4 + (in >> 4)) * tile_width(DIM, 2) : 0;
+}
+
+// Number of the tile at tile coordinates (x, y, z).
+template <int DIM>
+__device__ inline uint32_t tile_number(const TileList& l, uint32_t x, uint32_t y, uint32_t z) {
+  const uint32_t bx = (uint32_t)l.nt[0] / 4, by = (uint32_t)l.nt[1] / 4;
+  if (DIM == 2) return (x / 4 + bx * (y / 4)) * 16 + (x & 3) + 4 * (y & 3);
+  return (x / 4 + bx * (y / 4 + by * (z / 4))) * 64 + (x & 3) + 4 * (y & 3) + 16 * (z & 3);
+}
+
+// Grid offset of point (x, y, z), at its INVERSE-fftshifted position when
+// `shift` (std_gpuNUFFT_kernels.cu:629-654).
+template <int DIM>
+__device__ inline size_t tile_store_index(const Geom& g, int x, int y, int z, bool shift) {
+  if (shift) {
+    x = x < g.shift_inv[0] ? x - g.shift_inv[0] + g.G[0] : x - g.shift_inv[0];
+    y = y < g.shift_inv[1] ? y - g.shift_inv[1] + g.G[1] : y - g.shift_inv[1];
+    if (DIM == 3) z = z < g.shift_inv[2] ? z - g.shift_inv[2] + g.G[2] : z - g.shift_inv[2];
+  }
+  return (size_t)x + (size_t)g.G[0] * ((size_t)y + (DIM == 3 ? (size_t)g.G[1] * z : 0));
+}
+#endif
+
+// ---------------------------------------------------------------------------
 // Exact per-sample index / weight arithmetic. Contraction is disabled so the
 // float rounding of every ceil/floor/round input matches the reference's
 // separate multiply and add (CUDA/inc/gpuNUFFT_utils.hpp:89-104, 194-209).
@@ -98,6 +187,13 @@ __device__ __host__ inline float lerp_fetch(const float* tab, int K, float u) {
   return (1.0f - a) * tab[i0] + a * tab[i1];
 }
 
+// roundf(x) as an integer for x >= 0 (half away from zero), without the sign
+// handling of the library call.
+__device__ __host__ inline int round_index(float x) {
+  const int i = (int)x;
+  return x - (float)i >= 0.5f ? i + 1 : i;
+}
+
 // Weight of one tap along one axis; returns false when the nearest-mode
 // radius test rejects the tap (atomic_gpuNUFFT_kernels.cu:343-368); the
 // linear mode has no radius test (texture_gpuNUFFT_kernels.cu:63-82).
@@ -108,7 +204,7 @@ __device__ __host__ inline bool axis_weight(const Geom& g, const float* lut, int
   d *= d;
   if (g.lookup == 0) {
     if (!(d < g.rsq)) return false;
-    int li = (int)roundf(d * g.dist_mult);
+    int li = round_index(d * g.dist_mult);
     *w = lut[li < g.K - 1 ? li : g.K - 1];
     return true;
   }
@@ -124,7 +220,7 @@ __device__ __host__ inline bool axis_weight_kp(const Geom& g, const float* lut, 
   d *= d;
   if (g.lookup == 0) {
     if (!(d < g.rsq)) return false;
-    int li = (int)roundf(d * g.dist_mult);
+    int li = round_index(d * g.dist_mult);
     *w = lut[li < g.K - 1 ? li : g.K - 1];
     return true;
   }
@@ -189,7 +285,69 @@ hipError_t count_chunks(const uint32_t* sdc, uint32_t S, uint32_t chunk, uint32_
 hipError_t launch_fill_chunks(const uint32_t* sdc, const uint32_t* chunk_off, uint32_t S,
                               uint32_t chunk, Chunk* chunks, hipStream_t s);
 
+// Tap table of the sorted samples (s the caller's sample idx[s]), the square
+// roots of their density weights (dens NULL: none), both in the caller's
+// order, and per caller's sample the number of tiles its taps reach (counts).
+hipError_t launch_taps(const Geom& g, const float* crds, const float* dens, const uint32_t* idx, const float* lut,
+                       float4* taps, float* dens_sqrt, uint32_t* counts, hipStream_t s);
+// Exclusive sums of n counts (n + 1 of them).
+hipError_t scan_counts(void* temp, size_t* temp_bytes, const uint32_t* counts, uint64_t* offs, size_t n,
+                       hipStream_t s);
+// (tile, sample) pairs of every sample at its offset
+hipError_t launch_emit_pairs(const Geom& g, const TileList& l, const float4* taps, const uint64_t* offs,
+                             uint32_t* keys, uint32_t* vals, hipStream_t s);
+hipError_t sort_tile_pairs(void* temp, size_t* temp_bytes, const uint32_t* keys_in, uint32_t* keys_out,
+                           const uint32_t* vals_in, uint32_t* vals_out, size_t n, int key_bits, hipStream_t s);
+// the tiles' offsets in the sorted pairs (tiles + 1)
+hipError_t launch_tile_offsets(const uint32_t* keys, size_t n, uint32_t tiles, uint64_t* tile_off, hipStream_t s);
+// chunks of at most `chunk` entries: per-tile exclusive sums (tiles + 1)
+hipError_t scan_tile_chunks(void* temp, size_t* temp_bytes, const uint64_t* tile_off, uint32_t tiles,
+                            uint32_t chunk, TileTotals* tot, hipStream_t s);
+hipError_t fill_tile_chunks(const uint64_t* tile_off, uint32_t tiles, uint32_t chunk, const TileTotals* tot,
+                            TileChunk* chunks, TileTask* tasks, hipStream_t s);
+
+// All tables of a short trajectory (caller's order; short_tables_ok).
+struct ShortTables {
+  const float* traj;  // [dim][M]
+  const float* dens;  // NULL: none
+  const float* lut;
+  uint32_t S, n_tiles, chunk;  // sectors, tiles, samples per interp chunk
+  uint32_t max_slots;          // partial tiles
+  // sector tables
+  uint32_t *assigned, *idx, *sdc, *centers;
+  float *traj_sorted, *dens_sorted;
+  Chunk *chunks, *runs;  // room for S + M / chunk each
+  // tap table and tile lists
+  float4* taps;
+  float* dens_sqrt;
+  uint32_t* entries;       // room for every pair (short_tables_entries)
+  TileChunk* tile_chunks;  // room for n_tiles + entries / 128
+  TileTask* tile_tasks;    // room for n_tiles
+  uint32_t* host;          // pinned: sdc (S + 1 words), then chunks, runs, tile chunks, slots, tasks
+  uint32_t *counts, *offs;  // short_tables_words each
+};
+constexpr uint32_t kShortTotals = 5;
+bool short_tables_ok(uint32_t M, uint32_t S, uint32_t n_tiles);
+size_t short_tables_entries(const Geom& g, uint32_t M);
+size_t short_tables_words(uint32_t M, uint32_t S, uint32_t n_tiles);
+// temp NULL: only sets *temp_bytes
+hipError_t launch_short_tables(const Geom& g, const TileList& l, const ShortTables& t, void* temp,
+                               size_t* temp_bytes, hipStream_t s);
+// Entries per tile chunk for `pairs` list entries: enough chunks for the whole
+// device, between 128 and 512 (2-D) or 2048 (3-D).
+__device__ __host__ inline uint32_t tile_chunk(int dim, uint64_t pairs) {
+  const uint32_t most = dim == 3 ? 2048u : 512u;
+  uint32_t chunk = 128;
+  while (chunk < most && (uint64_t)chunk * 1024 < pairs) chunk *= 2;
+  return chunk;
+}
+
 // gridding.hip
+
+// Chunks per interp run: 4 stages the dense k-space centre's sectors fewer
+// times at the 128^3 koosh workload (interp 0.62 -> 0.60 ms); 8 and whole
+// sectors leave a long tail of busy workgroups (0.67 and 1.62 ms).
+constexpr int kInterpRun = 4;
 
 // Gridding work list: chunks in sector order, split into 8 contiguous
 // ranges of about equal cost; range x is processed on XCD x (workgroups
@@ -205,45 +363,28 @@ struct WorkList {
 // Split `n` chunks of the given sample counts into the 8 ranges of `w`.
 void partition_work(const uint32_t* counts, uint32_t n, WorkList* w);
 
-// Padded-sector coverage, per axis a: the home interval
-// [s*sw, min(s*sw + sw, G)) of sector index s along a meets (with periodic
-// wrap) the padded regions of the sector indices
-// ent[a][off[a][s] .. off[a][s+1]).
-struct Cover {
-  const uint32_t* off[3];
-  const uint32_t* ent[3];
-  int max_len[3];  // longest list per axis
-  // most (candidate, periodic image) pairs covering one grid coordinate of
-  // one axis; the fold indexes them per coordinate when at most kCovMax
-  int max_cov;
-};
-
-// Host: build the per-axis lists of `g` as one array (offsets of axis a at
-// word base[a], entries at word base[3 + a]); max_len[a] = longest list,
-// max_cov as in Cover.
-void build_cover(const Geom& g, std::vector<uint32_t>* words, size_t base[6], int max_len[3],
-                 int* max_cov);
-
 struct SpreadArgs {
-  const float2* data;      // [coil][...] samples
+  const float2* data;      // [coil][...] samples, caller's order
   long long coil_stride;   // elements between coils of `data`
-  const uint32_t* gather;  // NULL: data already in sector order
-  const float* dens;       // NULL: no density weighting (sorted order)
-  const float* crds;       // sorted SoA [dim][M]
-  WorkList work;
-  const float* lut;
-  float2* scratch;         // sub-grids [chunk][coil block][padded point][block width]
-  int sub_cb;              // coil block of that layout (the spread's; set by its launcher)
-  const uint32_t* sector_chunks;  // [S+1] first chunk of each sector
-  const uint2* reduce_tasks;      // (first chunk, count) of each multi-chunk sector
-  uint32_t n_reduce;
-  Cover cover;
+  const float* dens;       // square roots of the density weights, caller's order (NULL: none)
+  const float4* taps;      // tap table [dim][M]
+  TileList tiles;
+  float2* scratch;         // partial tiles [slot][coil][tile point]
   float2* grid;            // [coil][Ng], every point written (no prior zeroing)
   int n_coils;
   bool fold_shift;         // store at INVERSE-fftshifted positions
-  int lane_per_cu;         // lane kernels: workgroups per CU their coil block is sized for (0: default)
 };
-hipError_t launch_spread(const Geom& g, const SpreadArgs& a, int chunk, hipStream_t s);
+hipError_t launch_spread(const Geom& g, const SpreadArgs& a, hipStream_t s);
+// False for geometries whose padded sector does not fit the LDS of a CU (the
+// interp stages padded sectors; gridding.hip).
+bool spread_supported(const Geom& g);
+bool padded_sector_fits(const Geom& g, int cb);
+// samples in sector order (sample s is the caller's sorted[s]) -> out [coil][n]
+hipError_t launch_unsort(const float2* data, long long coil_stride, uint32_t n, int n_coils,
+                         const uint32_t* sorted, float2* out, hipStream_t s);
+// False when the padded sectors covering one sector are more than 256 (sector
+// widths far below the kernel width).
+bool sector_cover_ok(const Geom& g);
 
 struct InterpArgs {
   const float2* grid;      // [coil][Ng]
@@ -257,15 +398,11 @@ struct InterpArgs {
   float scale;             // 1 (kernel only) or 1/sqrt(Ng)
   int n_coils;
   bool fold_shift;         // read grid at FORWARD-fftshifted positions
-  int lane_per_cu;         // as in SpreadArgs
+  int lane_per_cu;         // lane kernels: workgroups per CU their coil block is sized for (0: default)
   // runs of up to kInterpRun consecutive chunks of one sector, for the
   // round-based interp (it stages a sector once per run; n_chunks 0: none)
   WorkList work_runs;
 };
-// Chunks per interp run: 4 stages the dense k-space centre's sectors fewer
-// times at the 128^3 koosh workload (interp 0.62 -> 0.60 ms); 8 and whole
-// sectors leave a long tail of busy workgroups (0.67 and 1.62 ms).
-constexpr int kInterpRun = 4;
 hipError_t launch_interp(const Geom& g, const InterpArgs& a, int chunk, hipStream_t s);
 
 
@@ -314,7 +451,6 @@ struct BatchOp {
   InterpArgs i;
   PostArgs post;
   PreArgs pre;
-  int R_spread;
   int R_interp;
 };
 
@@ -324,6 +460,23 @@ struct BatchList {
   uint32_t xcd_begin[9];
   uint32_t max_range;
 };
+
+#if defined(__HIPCC__)
+// Item of workgroup bid in a batch list (the XCD mapping of work_chunk);
+// false past the end of its XCD's range.
+__device__ inline bool batch_item(const BatchList& l, uint32_t bid, uint4* it) {
+  const uint32_t x = bid & 7u;
+  const uint32_t i = l.xcd_begin[x] + (bid >> 3);
+  if (i >= l.xcd_begin[x + 1]) return false;
+  const uint4 v = l.items[i];
+  // workgroup-uniform: scalar registers, so the item's plan descriptor is
+  // read with scalar loads (as vector values every descriptor field would
+  // take VGPRs)
+  *it = make_uint4(__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y),
+                   __builtin_amdgcn_readfirstlane(v.z), __builtin_amdgcn_readfirstlane(v.w));
+  return true;
+}
+#endif
 
 // Split items of the given costs into the 8 XCD ranges of `l` (items stay in order).
 void partition_items(const uint32_t* costs, uint32_t n, BatchList* l);
@@ -341,34 +494,27 @@ constexpr int kBatchThreads = 512;
 // chunks, and a 512-thread workgroup would leave most of its waves idle).
 constexpr int kBatchSmallThreads = 128;
 constexpr int kBatchPerCU = 4;
-hipError_t launch_spread_batch(int dim, int nx, const BatchOp* ops, const BatchList& l,
+// Spread of a batch: `items` (operator, chunk of its tile lists, coil group)
+// by coils per workgroup nc (nx: taps per axis, 4 or 8); tasks (operator, task, coil, block) of the tiles
+// with several chunks.
+hipError_t launch_spread_batch(int dim, int nx, int nc, const BatchOp* ops, const BatchList& l,
                                size_t lds, hipStream_t s);
-// generic: some plan's cover exceeds the fold's per-coordinate tables
-// (fold_generic), so the kernel variant with the generic body runs
-hipError_t launch_fold_batch(int dim, const BatchOp* ops, const BatchList& l, int threads,
-                             bool generic, hipStream_t s);
-bool fold_generic(const Cover& cover);
+hipError_t launch_tile_reduce_batch(int dim, const BatchOp* ops, const BatchList& tasks, hipStream_t s);
+size_t spread_lds_bytes(int dim, int nc);
 hipError_t launch_interp_batch(int dim, int nx, const BatchOp* ops, const BatchList& l,
                                size_t lds, hipStream_t s);
 // lane kernels in kBatchSmallThreads workgroups, for chunks of at most
 // 2 * kBatchSmallThreads samples
-hipError_t launch_spread_batch_small(int dim, const BatchOp* ops, const BatchList& l, size_t lds,
-                                     hipStream_t s);
 hipError_t launch_interp_batch_small(int dim, const BatchOp* ops, const BatchList& l, size_t lds,
                                      hipStream_t s);
-size_t spread_lds_bytes(const Geom& g, int cb, int R);
 // Batched lane kernels (launch_*_batch with nx == 3): usable for plan g;
 // their dynamic LDS for a coil block of cb.
 bool lane_batch_ok(const Geom& g);
-hipError_t launch_reduce_batch(const BatchOp* ops, const BatchList& l, uint32_t max_kstride,
-                               hipStream_t s);
-// lut: with the kernel table copied to LDS (the small-workgroup spread reads it from global memory)
+// lut: with the kernel table copied to LDS (small workgroups read it from global memory)
 size_t lane_lds_bytes(const Geom& g, int cb, bool lut = true);
 size_t interp_lds_bytes(const Geom& g, int cb, int R);
-int spread_round(const Geom& g, int cb, int chunk, size_t limit);
 int interp_round(const Geom& g, int cb, int chunk, size_t limit);
 size_t lds_budget();
-int fold_threads(const Geom& g, const Cover& cover);
 
 // prepost.hip: items (operator, block of 256 pixels / grid points, 0, 0)
 hipError_t launch_post_batch(const BatchOp* ops, const BatchList& l, hipStream_t s);

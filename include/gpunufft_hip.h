@@ -124,10 +124,10 @@ enum { GNUFFT_FFT_FUSED = 0, GNUFFT_FFT_ROCFFT = 1 };
 int gnufft_plan_set_fft(gnufft_plan plan, int kind);
 int gnufft_plan_get_fft(gnufft_plan plan, int* kind);
 
-/* Launch shape of a plan's kernel-width-3 gridding kernels. The reference
+/* Launch shape of a plan's kernel-width-3 interp. The reference
  * launches fixed 256-thread blocks, one per sector (THREAD_BLOCK_SIZE,
  * CUDA/inc/cuda_utils.cuh:75-77; getOptimalGridDim, cuda_utils.hpp:155).
- * Here the spread and interp workgroups size their coil block (4, 2 or 1
+ * Here the interp's workgroups size their coil block (4, 2 or 1
  * coils of a padded sector in LDS) for n workgroups per CU, falling back
  * to fewer when the sector does not fit: n = 0 restores the default (3, or
  * the GNUFFT_LANE_PER_CU environment variable), 1..8 sets it for this
@@ -203,7 +203,7 @@ int gnufft_adjoint(gnufft_plan plan, const void* kdata, void* out, uint32_t n_co
  * for callers that cannot allocate device memory (code under HIP graph
  * capture, serving loops, harnesses that forbid hipMalloc). Same arguments
  * and results as gnufft_adjoint; the plan (trajectory, sensitivities) must
- * be set up beforehand. The work grid and the spread sub-grids live in a
+ * be set up beforehand. The work grid and the spread's partial tiles live in a
  * fixed area of gnufft_noalloc_capacity() bytes (64 MiB) per device, a
  * static device array that each device holds until the process ends; coils
  * run in batches that fit it. Every call on a device shares that device's
@@ -258,9 +258,9 @@ int gnufft_interp_sorted(gnufft_plan plan, const void* grid, void* data_sorted,
  * balanced sector order of CUDA/src/gpuNUFFT_operator_factory.cpp:74-126).
  * A batch runs the full adjoint or forward of many plans (any image sizes
  * and trajectory lengths; one dimension and kernel-width class) with one
- * launch per stage: spread, chunk reduction, fold, post, pre and interp
- * kernels take (plan, work item, coil block) tiles from one list balanced
- * over the XCDs; FFTs run once per distinct grid size, batched over all
+ * launch per stage (the spread one per coil-group size): spread, tile
+ * reduction, post, pre and interp kernels take (plan, work item, coil block)
+ * items from lists balanced over the XCDs; FFTs run once per distinct grid size, batched over all
  * coils of those plans.
  * n_coils[i]: coils of plan i (its sensitivity coil count when it has
  * sensitivities). The batch keeps the plans' device tables by reference:
