@@ -242,14 +242,10 @@ struct gnufft_plan_s {
   Chunk* chunks_d = nullptr;
   uint32_t n_chunks = 0;
   uint32_t chunk = 1024;
-  // samples per LDS round of the gridding kernels: the mean chunk occupancy
-  // rounded up to 64 (sparse trajectories get small footprints, hence more
-  // workgroups per CU), at most `chunk`
-  uint32_t round_target = 1024;
   WorkList work{};
-  // the chunks of each sector merged in runs of up to kInterpRun (the
-  // round-based interp stages a sector once per run); empty when no sector
-  // has more than one chunk
+  // the chunks of each sector merged in runs of up to kInterpRun (the 3-D
+  // interp stages a sector once per run); empty when no sector has more than
+  // one chunk
   Chunk* runs_d = nullptr;
   WorkList work_runs{};
   int lane_per_cu = 0;  // gnufft_plan_set_workgroups_per_cu (0: default)
@@ -627,8 +623,6 @@ std::vector<Chunk> partition_chunks(gnufft_plan p, const uint32_t* sdc, uint32_t
   p->n_chunks = total;
   p->work.chunks = p->chunks_d;
   partition_work(counts.data(), total, &p->work);
-  const uint64_t mean = total ? ((uint64_t)p->M + total - 1) / total : 64;
-  p->round_target = (uint32_t)std::min<uint64_t>(p->chunk, std::max<uint64_t>(64, (mean + 63) / 64 * 64));
   const uint64_t run = (uint64_t)p->chunk * kInterpRun;
   for (uint32_t i = 0; i < p->S; i++)
     for (uint64_t b = sdc[i]; b < sdc[i + 1]; b += run) {
@@ -820,8 +814,7 @@ int build_short(gnufft_plan p, const float* traj, uint32_t M, const float* dens,
 
 bool valid_stop(int stop) { return stop >= 0 && stop <= 3; }
 
-// Spread arguments shared by every entry point: samples in sector order
-// (no gather, no density) unless the caller sets them.
+// Spread arguments shared by every entry point (no density).
 SpreadArgs spread_args(gnufft_plan p, const float2* data, float2* grid, uint32_t n_coils) {
   SpreadArgs a{};
   a.data = data;
@@ -831,6 +824,17 @@ SpreadArgs spread_args(gnufft_plan p, const float2* data, float2* grid, uint32_t
   a.scratch = p->scratch_d;
   a.grid = grid;
   a.n_coils = (int)n_coils;
+  return a;
+}
+
+// Interp arguments shared by every entry point.
+InterpArgs interp_args(gnufft_plan p) {
+  InterpArgs a{};
+  a.work = p->g.dim == 3 && p->work_runs.n_chunks ? p->work_runs : p->work;
+  a.taps = p->taps_d;
+  a.idx = p->idx_d;
+  a.coil_stride = p->M;
+  a.per_cu = p->lane_per_cu;
   return a;
 }
 
@@ -975,7 +979,7 @@ int gnufft_plan_create(gnufft_plan* plan, const uint32_t img_dims[3], uint32_t k
   }
   g.fft_scale = 1.0f / (float)std::sqrt((float)g.Ng);
   g.M = 0;
-  p->chunk = 1024;
+  p->chunk = g.dim == 3 ? 1024 : 256;
 
   p->lut = make_lut(K, kernel_width, osf);
   int rc = copy_in((void**)&p->lut_d, p->lut.data(), p->lut.size() * sizeof(float), GNUFFT_HOST, s);
@@ -1402,18 +1406,13 @@ int gnufft_interp_sorted(gnufft_plan p, const void* grid, void* data_sorted, uin
                          void* stream) {
   if (!p || !grid || (!data_sorted && p->M)) return fail(GNUFFT_ERR_INVALID_ARGUMENT, "interp_sorted: null");
   if (!p->sdc_d) return fail(GNUFFT_ERR_STATE, "interp_sorted: no trajectory set");
-  InterpArgs a{};
+  InterpArgs a = interp_args(p);
   a.grid = (const float2*)grid;
-  a.crds = p->traj_sorted_d;
-  a.work = p->work;
-  a.work_runs = p->work_runs;
-  a.lane_per_cu = p->lane_per_cu;
-  a.lut = p->lut_d;
   a.out = (float2*)data_sorted;
-  a.coil_stride = p->M;
+  a.sorted_out = true;
   a.scale = 1.0f;
   a.n_coils = (int)n_coils;
-  TIMED(p, GNUFFT_T_INTERP, (hipStream_t)stream, launch_interp(p->g, a, (int)p->round_target, (hipStream_t)stream));
+  TIMED(p, GNUFFT_T_INTERP, (hipStream_t)stream, launch_interp(p->g, a, (hipStream_t)stream));
   return GNUFFT_OK;
 }
 
@@ -1495,19 +1494,12 @@ int gnufft_forward(gnufft_plan p, const void* img, void* out, uint32_t n_coils, 
     }
     TIMED(p, GNUFFT_T_PREPOST, s, launch_image_prep(g, (const float2*)img, !use_sens, p->sens_d, p->deapo_d,
                               p->img_tmp_d, (int)n_coils, s));
-    InterpArgs a{};
+    InterpArgs a = interp_args(p);
     a.grid = p->img_tmp_d;
-    a.crds = p->traj_sorted_d;
-    a.work = p->work;
-    a.work_runs = p->work_runs;
-    a.lane_per_cu = p->lane_per_cu;
-    a.lut = p->lut_d;
     a.out = (float2*)out;
-    a.coil_stride = p->M;
-    a.scatter = p->idx_d;
     a.scale = 1.0f;
     a.n_coils = (int)n_coils;
-    TIMED(p, GNUFFT_T_INTERP, s, launch_interp(g, a, (int)p->round_target, s));
+    TIMED(p, GNUFFT_T_INTERP, s, launch_interp(g, a, s));
     return GNUFFT_OK;
   }
   const uint32_t cc = coil_batch(p, n_coils);
@@ -1531,21 +1523,14 @@ int gnufft_forward(gnufft_plan p, const void* img, void* out, uint32_t n_coils, 
       rc = run_fft(p, nc, false, p->grid_d, s);
       if (rc) return rc;
     }
-    InterpArgs a{};
+    InterpArgs a = interp_args(p);
     a.grid = p->grid_d;
-    a.crds = p->traj_sorted_d;
-    a.work = p->work;
-    a.work_runs = p->work_runs;
-    a.lane_per_cu = p->lane_per_cu;
-    a.lut = p->lut_d;
     a.out = (float2*)out + (size_t)c0 * p->M;
-    a.coil_stride = p->M;
-    a.scatter = p->idx_d;
-    a.dens = p->dens_sorted_d;
+    a.dens = p->dens_sqrt_d;
     a.scale = g.fft_scale;
     a.n_coils = (int)nc;
     a.fold_shift = true;
-    TIMED(p, GNUFFT_T_INTERP, s, launch_interp(g, a, (int)p->round_target, s));
+    TIMED(p, GNUFFT_T_INTERP, s, launch_interp(g, a, s));
   }
   return GNUFFT_OK;
 }
@@ -1556,6 +1541,7 @@ int gnufft_forward(gnufft_plan p, const void* img, void* out, uint32_t n_coils, 
 }  // extern "C"
 
 constexpr int kSpreadNc[3] = {2, 4, 8};  // coil-group sizes of the batched spread
+constexpr int kInterpNc[4] = {1, 2, 4, 8};
 
 struct gnufft_batch_s {
   int dim = 2, nx = 4;
@@ -1566,10 +1552,11 @@ struct gnufft_batch_s {
   std::vector<BatchOp> ops_h;
   BatchOp* ops_d = nullptr;
   uint4* items_d = nullptr;
-  // spread: one list per coil-group size (kSpreadNc); interp, lane kernels:
-  // chunks of at most 2 * kBatchSmallThreads samples run in small workgroups
-  BatchList spread[3]{}, reduce{}, interp{}, interp_small{}, post{}, pre{};
-  size_t spread_lds[3] = {0, 0, 0}, interp_lds = 0, interp_small_lds = 0;
+  // one list per coil-group size (kSpreadNc, kInterpNc)
+  BatchList spread[3]{}, reduce{}, interp[4]{}, post{}, pre{};
+  size_t spread_lds[3] = {0, 0, 0}, interp_lds[4] = {0, 0, 0, 0};
+  int taps = 3;  // of the interp kernels
+  bool full_taps = true;
   float2* grid_d = nullptr;
   float2* scratch_d = nullptr;
   struct Group {
@@ -1681,12 +1668,11 @@ int gnufft_batch_create(gnufft_batch* batch, const gnufft_plan* plans, uint32_t 
   auto batch_fused = [](const gnufft_plan q) { return q->fused && fused_fft_supported(q->g); };
   b->dim = g0.dim;
   b->nx = nx;
-  // kernel width 3 in every plan: the lane kernels (tap records in
-  // registers), flagged as nx = 3 for the batched launchers
-  bool lane = true;
-  for (uint32_t i = 0; i < n_plans; i++) lane = lane && lane_batch_ok(plans[i]->g);
-  if (lane) b->nx = 3;
-  const uint32_t grid_cb = lane ? (uint32_t)kBatchLaneCB : (uint32_t)kBatchCB;
+  // interp kernels for the widest plan
+  b->taps = 3;
+  for (uint32_t i = 0; i < n_plans; i++) b->taps = std::max(b->taps, interp_taps(plans[i]->g.kw));
+  b->full_taps = true;
+  for (uint32_t i = 0; i < n_plans; i++) b->full_taps = b->full_taps && plans[i]->g.kw == b->taps;
   b->fused = false;
   b->fft_prime = false;
   for (uint32_t i = 0; i < n_plans; i++) {
@@ -1702,19 +1688,6 @@ int gnufft_batch_create(gnufft_batch* batch, const gnufft_plan* plans, uint32_t 
     if (ga.G[1] != gc.G[1]) return ga.G[1] < gc.G[1];
     return ga.G[0] < gc.G[0];
   });
-  // One launch per stage uses the largest footprint of any plan, so each
-  // plan's round size is the largest that still lets kBatchPerCU workgroups
-  // share a CU (then fewer): one dense plan must not cut the occupancy of
-  // the whole batch.
-  auto batch_round = [](int (*round)(const Geom&, int, int, size_t), const Geom& g, int target,
-                        size_t reserve) {
-    const int need = std::min(64, target);
-    for (int k = kBatchPerCU; k >= 1; k--) {
-      const int r = round(g, kBatchCB, target, lds_budget() / k - 1024 - reserve);
-      if (r >= need || (k == 1 && r > 0)) return r;
-    }
-    return 0;
-  };
   size_t grid_total = 0, scratch_total = 0;
   std::vector<size_t> grid_off(n_plans), scratch_off(n_plans);
   for (uint32_t k = 0; k < n_plans; k++) {
@@ -1747,27 +1720,23 @@ int gnufft_batch_create(gnufft_batch* batch, const gnufft_plan* plans, uint32_t 
     return fail(GNUFFT_ERR_OUT_OF_MEMORY, "batch_create: grid / scratch allocation");
   }
   // descriptors and item lists
-  // spread items (tile chunk, coil group) by group size; interp items (chunk,
-  // coil block) of large (il) and small (is) chunks
-  std::vector<uint4> sp[3], il, is, rd, po, pr;
-  std::vector<uint32_t> sp_cost[3], il_cost, is_cost;
+  // spread items (tile chunk, coil group) and interp items (chunk, coil group)
+  // by group size
+  std::vector<uint4> sp[3], il[4], rd, po, pr;
+  std::vector<uint32_t> sp_cost[3], il_cost[4];
   for (uint32_t k = 0; k < n_plans && !rc; k++) {
     const gnufft_plan p = b->plans[k];
     const uint32_t C = b->coils[k];
-    const uint32_t cbs = (C + grid_cb - 1) / grid_cb;  // interp coil blocks
     BatchOp op{};
     op.g = p->g;
     op.s = spread_args(p, nullptr, b->grid_d + grid_off[k], C);
     op.s.scratch = b->scratch_d + scratch_off[k];
     op.s.dens = p->dens_sqrt_d;
     op.s.fold_shift = true;
+    op.i = interp_args(p);
     op.i.grid = b->grid_d + grid_off[k];
-    op.i.crds = p->traj_sorted_d;
-    op.i.work = p->work;
-    op.i.lut = p->lut_d;
-    op.i.coil_stride = p->M;
-    op.i.scatter = p->idx_d;
-    op.i.dens = p->dens_sorted_d;
+    op.i.dens = p->dens_sqrt_d;
+    op.i.row_bits = interp_row_bits(p->g);
     op.i.scale = p->g.fft_scale;
     op.i.n_coils = (int)C;
     op.i.fold_shift = true;
@@ -1775,17 +1744,14 @@ int gnufft_batch_create(gnufft_batch* batch, const gnufft_plan* plans, uint32_t 
                        p->n_sens ? p->sens_d : nullptr, nullptr, GNUFFT_STOP_DEAPODIZATION};
     op.pre = PreArgs{nullptr, p->n_sens ? 0 : 1, p->n_sens ? p->sens_d : nullptr, p->deapo_d,
                      b->grid_d + grid_off[k], (int)C};
-    op.R_interp = batch_round(interp_round, p->g, (int)p->round_target, 3072);
-    if (!padded_sector_fits(p->g, kBatchCB) || op.R_interp <= 0) {
+    int iq = 0;
+    const int inc = interp_coils(p->g, (int)C, p->lane_per_cu);
+    if (!batch_sector_fits(p->g, kBatchCB) || inc == 0) {
       rc = fail(GNUFFT_ERR_UNSUPPORTED, "batch_create: padded sector does not fit in LDS");
       break;
     }
-    if (lane) {
-      b->interp_small_lds = std::max(b->interp_small_lds, lane_lds_bytes(p->g, kBatchLaneCB, false));
-      b->interp_lds = std::max(b->interp_lds, lane_lds_bytes(p->g, kBatchLaneCB));
-    } else {
-      b->interp_lds = std::max(b->interp_lds, interp_lds_bytes(p->g, kBatchCB, op.R_interp));
-    }
+    while (kInterpNc[iq] < inc) iq++;
+    b->interp_lds[iq] = std::max(b->interp_lds[iq], interp_lds_bytes(p->g, inc, b->taps));
     if (!p->cover_ok) {
       rc = fail(GNUFFT_ERR_UNSUPPORTED, "batch_create: too many sectors cover a point");
       break;
@@ -1802,22 +1768,19 @@ int gnufft_batch_create(gnufft_batch* batch, const gnufft_plan* plans, uint32_t 
       }
     }
     // chunk lists (host copies) for the gridding items and the reduce tasks
-    std::vector<Chunk> ch(p->n_chunks);
+    std::vector<Chunk> ch(op.i.work.n_chunks);
     std::vector<TileChunk> tc(p->tiles.n_chunks);
-    if ((p->n_chunks &&
-         hipMemcpy(ch.data(), p->chunks_d, ch.size() * sizeof(Chunk), hipMemcpyDeviceToHost) != hipSuccess) ||
+    if ((!ch.empty() &&
+         hipMemcpy(ch.data(), op.i.work.chunks, ch.size() * sizeof(Chunk), hipMemcpyDeviceToHost) != hipSuccess) ||
         hipMemcpy(tc.data(), p->tile_chunks_d, tc.size() * sizeof(TileChunk), hipMemcpyDeviceToHost) != hipSuccess) {
       rc = fail(GNUFFT_ERR_DEVICE, "batch_create: chunk list copy");
       break;
     }
-    for (uint32_t ci = 0; ci < p->n_chunks; ci++) {
-      const uint32_t n = ch[ci].end - ch[ci].begin;
-      const bool small = lane && n <= 2u * (uint32_t)kBatchSmallThreads;
-      for (uint32_t cb = 0; cb < cbs; cb++) {
-        (small ? is : il).push_back(make_uint4(k, ci, cb, 0));
-        (small ? is_cost : il_cost).push_back(n + (small ? 100u : 300u));
+    for (uint32_t ci = 0; ci < (uint32_t)ch.size(); ci++)
+      for (uint32_t cg = 0; cg * kInterpNc[iq] < C; cg++) {
+        il[iq].push_back(make_uint4(k, ci, cg, 0));
+        il_cost[iq].push_back(ch[ci].end - ch[ci].begin + 100u);
       }
-    }
     int q = 0;
     while (kSpreadNc[q] < tile_coils((int)C)) q++;
     b->spread_lds[q] = spread_lds_bytes(p->g.dim, kSpreadNc[q]);
@@ -1838,8 +1801,7 @@ int gnufft_batch_create(gnufft_batch* batch, const gnufft_plan* plans, uint32_t 
   if (!rc) {
     std::vector<uint4> all;
     for (auto& v : sp) all.insert(all.end(), v.begin(), v.end());
-    all.insert(all.end(), il.begin(), il.end());
-    all.insert(all.end(), is.begin(), is.end());
+    for (auto& v : il) all.insert(all.end(), v.begin(), v.end());
     all.insert(all.end(), rd.begin(), rd.end());
     all.insert(all.end(), po.begin(), po.end());
     all.insert(all.end(), pr.begin(), pr.end());
@@ -1863,8 +1825,7 @@ int gnufft_batch_create(gnufft_batch* batch, const gnufft_plan* plans, uint32_t 
       at += v.size();
     };
     for (int q = 0; q < 3; q++) list(b->spread[q], sp[q], &sp_cost[q]);
-    list(b->interp, il, &il_cost);
-    list(b->interp_small, is, &is_cost);
+    for (int q = 0; q < 4; q++) list(b->interp[q], il[q], &il_cost[q]);
     list(b->reduce, rd, nullptr);
     list(b->post, po, nullptr);
     list(b->pre, pr, nullptr);
@@ -1997,8 +1958,8 @@ int gnufft_batch_forward(gnufft_batch b, const void* const* img, void* const* ou
                                      b->fft_fwd_big[ps].lds, s));
     }
   }
-  HIP_TRY(launch_interp_batch(b->dim, b->nx, b->ops_d, b->interp, b->interp_lds, s));
-  HIP_TRY(launch_interp_batch_small(b->dim, b->ops_d, b->interp_small, b->interp_small_lds, s));
+  for (int q = 0; q < 4; q++)
+    HIP_TRY(launch_interp_batch(b->dim, kInterpNc[q], b->taps, b->full_taps, b->ops_d, b->interp[q], b->interp_lds[q], s));
   return batch_mark_done(b, s);
 }
 

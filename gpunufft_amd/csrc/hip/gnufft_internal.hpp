@@ -388,23 +388,20 @@ bool sector_cover_ok(const Geom& g);
 
 struct InterpArgs {
   const float2* grid;      // [coil][Ng]
-  const float* crds;
   WorkList work;
-  const float* lut;
-  float2* out;             // [coil][...]
+  const float4* taps;      // tap table [dim][M]
+  const uint32_t* idx;     // caller's number of sorted sample s
+  float2* out;             // [coil][...], caller's order
   long long coil_stride;
-  const uint32_t* scatter; // NULL: write in sector order
-  const float* dens;       // NULL: no density weighting
+  bool sorted_out;         // write in sector order
+  const float* dens;       // square roots of the density weights, caller's order (NULL: none)
   float scale;             // 1 (kernel only) or 1/sqrt(Ng)
   int n_coils;
   bool fold_shift;         // read grid at FORWARD-fftshifted positions
-  int lane_per_cu;         // lane kernels: workgroups per CU their coil block is sized for (0: default)
-  // runs of up to kInterpRun consecutive chunks of one sector, for the
-  // round-based interp (it stages a sector once per run; n_chunks 0: none)
-  WorkList work_runs;
+  int per_cu;              // workgroups per CU the coil group is sized for (0: default)
+  int row_bits;            // interp_row_bits (launch_interp sets it)
 };
-hipError_t launch_interp(const Geom& g, const InterpArgs& a, int chunk, hipStream_t s);
-
+hipError_t launch_interp(const Geom& g, const InterpArgs& a, hipStream_t s);
 
 // prepost.hip
 hipError_t launch_zero(void* p, size_t bytes, hipStream_t s);
@@ -451,7 +448,6 @@ struct BatchOp {
   InterpArgs i;
   PostArgs post;
   PreArgs pre;
-  int R_interp;
 };
 
 struct BatchList {
@@ -482,18 +478,8 @@ __device__ inline bool batch_item(const BatchList& l, uint32_t bid, uint4* it) {
 void partition_items(const uint32_t* costs, uint32_t n, BatchList* l);
 
 // gridding.hip (CB: coils per workgroup, the same for every operator).
-// Batched spread / interp workgroups have kBatchThreads threads and their
-// rounds are sized so that kBatchPerCU of them share a CU. (Smaller
-// workgroups do not raise that count: the 8-coil sub-grid dominates the LDS
-// footprint, 20.7 KB at 2-D sw 16.)
+// Coil block that a batch's padded sectors have to fit the LDS for.
 constexpr int kBatchCB = 8;
-constexpr int kBatchLaneCB = 4;  // coil block of the batched lane (kernel width 3) kernels
-constexpr int kBatchThreads = 512;
-// Batched lane kernels: chunks of at most 2 * kBatchSmallThreads samples run
-// in workgroups of kBatchSmallThreads (sparse 2-D plans are mostly such
-// chunks, and a 512-thread workgroup would leave most of its waves idle).
-constexpr int kBatchSmallThreads = 128;
-constexpr int kBatchPerCU = 4;
 // Spread of a batch: `items` (operator, chunk of its tile lists, coil group)
 // by coils per workgroup nc (nx: taps per axis, 4 or 8); tasks (operator, task, coil, block) of the tiles
 // with several chunks.
@@ -501,20 +487,18 @@ hipError_t launch_spread_batch(int dim, int nx, int nc, const BatchOp* ops, cons
                                size_t lds, hipStream_t s);
 hipError_t launch_tile_reduce_batch(int dim, const BatchOp* ops, const BatchList& tasks, hipStream_t s);
 size_t spread_lds_bytes(int dim, int nc);
-hipError_t launch_interp_batch(int dim, int nx, const BatchOp* ops, const BatchList& l,
+// taps, full: interp_taps of the widest plan, and whether every plan's kernel
+// width is that
+hipError_t launch_interp_batch(int dim, int nc, int taps, bool full, const BatchOp* ops, const BatchList& l,
                                size_t lds, hipStream_t s);
-// lane kernels in kBatchSmallThreads workgroups, for chunks of at most
-// 2 * kBatchSmallThreads samples
-hipError_t launch_interp_batch_small(int dim, const BatchOp* ops, const BatchList& l, size_t lds,
-                                     hipStream_t s);
-// Batched lane kernels (launch_*_batch with nx == 3): usable for plan g;
-// their dynamic LDS for a coil block of cb.
-bool lane_batch_ok(const Geom& g);
-// lut: with the kernel table copied to LDS (small workgroups read it from global memory)
-size_t lane_lds_bytes(const Geom& g, int cb, bool lut = true);
-size_t interp_lds_bytes(const Geom& g, int cb, int R);
-int interp_round(const Geom& g, int cb, int chunk, size_t limit);
-size_t lds_budget();
+int interp_taps(int kw);
+// log2 of the threads per staged row: a power of two, two points each
+int interp_row_bits(const Geom& g);
+// Coils per group (8, 4, 2, 1) of an interp launch; 0: the sector does not fit
+int interp_coils(const Geom& g, int n_coils, int per_cu);
+size_t interp_lds_bytes(const Geom& g, int nc, int taps);
+// The padded sector of `cb` coils fits a batch's LDS
+bool batch_sector_fits(const Geom& g, int cb);
 
 // prepost.hip: items (operator, block of 256 pixels / grid points, 0, 0)
 hipError_t launch_post_batch(const BatchOp* ops, const BatchList& l, hipStream_t s);
