@@ -44,6 +44,22 @@ constexpr int kPerThread = kTileElems / kFftThreads;  // tile elements per threa
 // tile of 16 lines (one workgroup per CU), the same work per thread
 constexpr int kBigThreads = 1024;
 constexpr int kBigTileElems = kPerThread * kBigThreads;
+// Light kernels, for transforms that leave the device short of tiles (2-D
+// grids): 8 elements per thread instead of 16 and as many threads as the tile
+// needs; 8 lines per tile of a y / z pass, and of an x pass as few image lines as
+// give 512 tiles. What bounds these passes is the chain of stages in a
+// workgroup (the 22 MB of a 480^2 grid with 12 coils would take 5 us), which
+// half the work per thread shortens. Adjoint and forward transform, full tiles
+// and light: 64^2 osf 2, 1 coil 15.9 -> 12.8 us each; 224^2 osf 1.5, 12 coils
+// 30.3 -> 25.5; 256^2 osf 2, 16 coils 36.1 -> 35.1; 240^2 osf 2, 12 coils
+// 33.0 -> 31.3. With many tiles the wider rows of the full tile win: 315 us
+// (full) and 483 us (light) at 192^3, 8 coils. Lengths with kernels of their own
+// (constant strides) keep them down to one tile per CU: x passes of 512 points
+// take 18 and 16 us, light ones 21 and 18.
+constexpr int kLightPerThread = 8;
+constexpr int kLightStripe = 8;
+constexpr uint32_t kLightBlocks = 2048, kLightX = 512;  // tiles of a y / z and of an x pass
+constexpr uint32_t kLightFixed = 256;                   // line lengths with kernels of their own
 constexpr int kMaxStripe = 32;    // lines per tile of a y / z pass (256 B rows)
 constexpr int kMaxPix = 4;        // image pixels per thread in the x passes
 constexpr int kMaxLen = kMaxPix * kFftThreads;  // longest transform (2048)
@@ -212,9 +228,10 @@ struct FftRadices {
   FftStage st[12];
 };
 
-template <int R>
+// PT: tile elements per thread
+template <int R, int PT>
 struct Bfly {
-  static constexpr int KB = (kPerThread + R - 1) / R;  // butterflies per thread
+  static constexpr int KB = (PT + R - 1) / R;  // butterflies per thread
 };
 
 // Twiddle, radix-R DFT and store of butterfly j (values v) at
@@ -243,10 +260,10 @@ __device__ __forceinline__ void finish_butterfly(float2* v, int j, int l, const 
 // Stage with its inputs fetched by get(l, index) and outputs stored by
 // put(l, index, value); a barrier separates all fetches from all stores
 // when `sync` (in-place LDS stages).
-template <int R, int NT = kFftThreads, typename Get, typename Put>
+template <int R, int NT = kFftThreads, int PT = kPerThread, typename Get, typename Put>
 __device__ __forceinline__ void stage(int lines, uint32_t m_lines, const FftStage& st, const float2* tw,
                              float sign, bool sync, Get get, Put put) {
-  constexpr int KB = Bfly<R>::KB;
+  constexpr int KB = Bfly<R, PT>::KB;
   const int B = lines * st.per_line;
   float2 v[KB][R];
 #pragma unroll
@@ -273,26 +290,26 @@ __device__ __forceinline__ void stage(int lines, uint32_t m_lines, const FftStag
 
 // PR: also the prime radices 7 .. 19 (their registers would otherwise set
 // the occupancy of every table-driven pass).
-template <int NT = kFftThreads, bool PR = false, typename Get, typename Put>
+template <int NT, int PT, bool PR, typename Get, typename Put>
 __device__ __forceinline__ void stage_any(int lines, uint32_t m_lines, const FftStage& table_entry,
                                  const float2* tw, float sign, bool sync, Get get, Put put) {
   // a register copy: the table lives in global memory, and stores of the
   // stage to global memory would otherwise force reloads of its fields
   const FftStage st = table_entry;
   switch (st.R) {
-    case 8: stage<8, NT>(lines, m_lines, st, tw, sign, sync, get, put); break;
-    case 4: stage<4, NT>(lines, m_lines, st, tw, sign, sync, get, put); break;
-    case 2: stage<2, NT>(lines, m_lines, st, tw, sign, sync, get, put); break;
-    case 3: stage<3, NT>(lines, m_lines, st, tw, sign, sync, get, put); break;
-    case 5: stage<5, NT>(lines, m_lines, st, tw, sign, sync, get, put); break;
+    case 8: stage<8, NT, PT>(lines, m_lines, st, tw, sign, sync, get, put); break;
+    case 4: stage<4, NT, PT>(lines, m_lines, st, tw, sign, sync, get, put); break;
+    case 2: stage<2, NT, PT>(lines, m_lines, st, tw, sign, sync, get, put); break;
+    case 3: stage<3, NT, PT>(lines, m_lines, st, tw, sign, sync, get, put); break;
+    case 5: stage<5, NT, PT>(lines, m_lines, st, tw, sign, sync, get, put); break;
     default:
       if constexpr (PR) {
         switch (st.R) {
-          case 7: stage<7, NT>(lines, m_lines, st, tw, sign, sync, get, put); break;
-          case 11: stage<11, NT>(lines, m_lines, st, tw, sign, sync, get, put); break;
-          case 13: stage<13, NT>(lines, m_lines, st, tw, sign, sync, get, put); break;
-          case 17: stage<17, NT>(lines, m_lines, st, tw, sign, sync, get, put); break;
-          default: stage<19, NT>(lines, m_lines, st, tw, sign, sync, get, put); break;
+          case 7: stage<7, NT, PT>(lines, m_lines, st, tw, sign, sync, get, put); break;
+          case 11: stage<11, NT, PT>(lines, m_lines, st, tw, sign, sync, get, put); break;
+          case 13: stage<13, NT, PT>(lines, m_lines, st, tw, sign, sync, get, put); break;
+          case 17: stage<17, NT, PT>(lines, m_lines, st, tw, sign, sync, get, put); break;
+          default: stage<19, NT, PT>(lines, m_lines, st, tw, sign, sync, get, put); break;
         }
       }
       break;
@@ -301,13 +318,13 @@ __device__ __forceinline__ void stage_any(int lines, uint32_t m_lines, const Fft
 
 // Transform `lines` lines held in LDS (stride LP) in place. Callers
 // synchronise after filling the lines; every stage ends with a barrier.
-template <bool PR>
+template <int NT, int PT, bool PR>
 __device__ __forceinline__ void fft_lines(float2* buf, int lines, uint32_t m_lines, int LP,
                                  const FftStage* st, int n_st, const float2* tw, float sign) {
   auto get = [&](int l, int i) { return buf[l * LP + i]; };
   auto put = [&](int l, int i, float2 v) { buf[l * LP + i] = v; };
   for (int i = 0; i < n_st; i++) {
-    stage_any<kFftThreads, PR>(lines, m_lines, st[i], tw, sign, true, get, put);
+    stage_any<NT, PT, PR>(lines, m_lines, st[i], tw, sign, true, get, put);
     __syncthreads();
   }
 }
@@ -349,18 +366,20 @@ __device__ __forceinline__ void fixed_middle(int lines, uint32_t m_lines, const 
 }
 
 // Stage runners: all stages of `lines` LDS lines (the x passes).
-template <bool PR>
+template <bool PR, int NT = kFftThreads, int PT = kPerThread>
 struct RunTable {
+  static constexpr int threads = NT;
   const FftStage* st;
   int n;
   __device__ __forceinline__ void operator()(float2* buf, int lines, uint32_t m_lines, int LP,
                                              const float2* tw, float sign) const {
-    fft_lines<PR>(buf, lines, m_lines, LP, st, n, tw, sign);
+    fft_lines<NT, PT, PR>(buf, lines, m_lines, LP, st, n, tw, sign);
   }
 };
 
 template <int L, int... R>
 struct RunFixed {
+  static constexpr int threads = kFftThreads;
   __device__ __forceinline__ void operator()(float2* buf, int lines, uint32_t m_lines, int LP,
                                              const float2* tw, float sign) const {
     using F = FixedStages<L, R...>;
@@ -396,6 +415,7 @@ struct AxisPass {
   int out_gather, out_off;
   int stripe, x_tiles, coils;
   int big;  // 1: lines above 511 points, kBigThreads and a kBigTileElems tile
+  int light;  // threads of the light kernel, 0: not used
   uint32_t m_stripe;
   float sign;
   const FftStage* st;  // stage table in device memory (beside the twiddles)
@@ -403,7 +423,7 @@ struct AxisPass {
   const float2* tw;
 };
 
-template <int NT, bool PR>
+template <int NT, bool PR, int PT = kPerThread>
 __device__ __forceinline__ void fft_axis_body(const AxisPass& p, int block) {
   extern __shared__ float2 lds[];
   float2* tw = lds;
@@ -441,16 +461,16 @@ __device__ __forceinline__ void fft_axis_body(const AxisPass& p, int block) {
   const int n = p.n_st;
   __syncthreads();  // twiddles
   if (n == 1) {
-    stage_any<NT, PR>(S, p.m_stripe, p.st[0], tw, p.sign, false, get_global, put_global);
+    stage_any<NT, PT, PR>(S, p.m_stripe, p.st[0], tw, p.sign, false, get_global, put_global);
     return;
   }
-  stage_any<NT, PR>(S, p.m_stripe, p.st[0], tw, p.sign, false, get_global, put_lds);
+  stage_any<NT, PT, PR>(S, p.m_stripe, p.st[0], tw, p.sign, false, get_global, put_lds);
   __syncthreads();
   for (int i = 1; i < n - 1; i++) {
-    stage_any<NT, PR>(S, p.m_stripe, p.st[i], tw, p.sign, true, get_lds, put_lds);
+    stage_any<NT, PT, PR>(S, p.m_stripe, p.st[i], tw, p.sign, true, get_lds, put_lds);
     __syncthreads();
   }
-  stage_any<NT, PR>(S, p.m_stripe, p.st[n - 1], tw, p.sign, false, get_lds, put_global);
+  stage_any<NT, PT, PR>(S, p.m_stripe, p.st[n - 1], tw, p.sign, false, get_lds, put_global);
 }
 
 template <bool PR>
@@ -461,6 +481,11 @@ __global__ void __launch_bounds__(kFftThreads, 4) fft_axis_kernel(AxisPass p) {
 template <bool PR>
 __global__ void __launch_bounds__(kBigThreads, 1) fft_axis_big_kernel(AxisPass p) {
   fft_axis_body<kBigThreads, PR>(p, blockIdx.x);
+}
+
+template <int NT, bool PR>
+__global__ void __launch_bounds__(NT, PR ? 4 : 8) fft_axis_light_kernel(AxisPass p) {
+  fft_axis_body<NT, PR, kLightPerThread>(p, blockIdx.x);
 }
 
 // The same pass for a line length L = R0 R1 ... (two or more stages) and a
@@ -527,6 +552,7 @@ struct LastPass {
   int crop0, shift0;
   int coils, Cg, Q;
   uint32_t m_g0, m_n0;  // qdiv constants for G0, N0
+  int light;            // threads of the light kernel, 0: not used
   float scale;
   int apply_deapo, accumulate;
   float sign;
@@ -537,12 +563,13 @@ struct LastPass {
 
 template <typename Run>
 __device__ __forceinline__ void fft_adjoint_last_body(const LastPass& p, int block, const Run& run) {
+  constexpr int NT = Run::threads;
   extern __shared__ float2 lds[];
   float2* tw = lds;
   float2* buf = lds + p.G0;
   const int l0 = block * p.Q;
   const int nq = min(p.Q, p.lines - l0);
-  for (int i = threadIdx.x; i < p.G0; i += kFftThreads) tw[i] = p.tw[i];
+  for (int i = threadIdx.x; i < p.G0; i += NT) tw[i] = p.tw[i];
   const long long Ni = (long long)p.N0 * p.lines;
   const long long cin = (long long)p.G0 * p.lines;
   const long long pix0 = (long long)l0 * p.N0;
@@ -558,11 +585,11 @@ __device__ __forceinline__ void fft_adjoint_last_body(const LastPass& p, int blo
       const int total = ng * per_coil;
       const uint32_t m_pc = qdiv_const_dev(per_coil);
       const float2* src = p.in + (long long)c0 * cin + (long long)l0 * p.G0;
-      for (int e0 = threadIdx.x; e0 < total; e0 += kTileLoads * kFftThreads) {
+      for (int e0 = threadIdx.x; e0 < total; e0 += kTileLoads * NT) {
         float2 v[kTileLoads];
 #pragma unroll
         for (int u = 0; u < kTileLoads; u++) {
-          const int e = e0 + u * kFftThreads;
+          const int e = e0 + u * NT;
           if (e < total) {
             const int c = qdiv(e, m_pc);
             v[u] = src[(long long)c * cin + (e - c * per_coil)];
@@ -570,7 +597,7 @@ __device__ __forceinline__ void fft_adjoint_last_body(const LastPass& p, int blo
         }
 #pragma unroll
         for (int u = 0; u < kTileLoads; u++) {
-          const int e = e0 + u * kFftThreads;
+          const int e = e0 + u * NT;
           if (e < total) {
             const int c = qdiv(e, m_pc);
             const int r = e - c * per_coil;
@@ -585,7 +612,7 @@ __device__ __forceinline__ void fft_adjoint_last_body(const LastPass& p, int blo
     // the coil sum of later coil groups (and of later calls when
     // accumulating) adds to what this thread wrote for the same pixels
     const bool add = c0 > 0 || p.accumulate;
-    for (int e = threadIdx.x; e < npix; e += kFftThreads) {
+    for (int e = threadIdx.x; e < npix; e += NT) {
       const int q = qdiv(e, p.m_n0);
       const int x = e - q * p.N0;
       const long long pix = pix0 + e;
@@ -641,6 +668,7 @@ struct FirstPass {
   int crop0, shift0;
   int coils, Cg, Q;
   uint32_t m_g0, m_n0, m_pad;  // qdiv constants for G0, N0, G0 - N0
+  int light;                   // threads of the light kernel, 0: not used
   float sign;
   const FftStage* st;  // stage table in device memory (beside the twiddles)
   int n_st;
@@ -649,12 +677,13 @@ struct FirstPass {
 
 template <typename Run>
 __device__ __forceinline__ void fft_forward_first_body(const FirstPass& p, int block, const Run& run) {
+  constexpr int NT = Run::threads;
   extern __shared__ float2 lds[];
   float2* tw = lds;
   float2* buf = lds + p.G0;
   const int l0 = block * p.Q;
   const int nq = min(p.Q, p.lines - l0);
-  for (int i = threadIdx.x; i < p.G0; i += kFftThreads) tw[i] = p.tw[i];
+  for (int i = threadIdx.x; i < p.G0; i += NT) tw[i] = p.tw[i];
   const long long Ni = (long long)p.N0 * p.lines;
   const long long cout = (long long)p.G0 * p.lines;
   const long long pix0 = (long long)l0 * p.N0;
@@ -665,12 +694,12 @@ __device__ __forceinline__ void fft_forward_first_body(const FirstPass& p, int b
     __syncthreads();  // the previous group's reads of buf are done
     // zero padding: positions of "pixels" N0 .. G0-1 of every line
     const int pad = p.G0 - p.N0;
-    for (int e = threadIdx.x; e < ng * nq * pad; e += kFftThreads) {
+    for (int e = threadIdx.x; e < ng * nq * pad; e += NT) {
       const int l = qdiv(e, p.m_pad);
       const int x = p.N0 + e - l * pad;
       buf[l * p.LP + wrap1(x + p.crop0 - p.shift0, p.G0)] = make_float2(0.f, 0.f);
     }
-    for (int e = threadIdx.x; e < npix; e += kFftThreads) {
+    for (int e = threadIdx.x; e < npix; e += NT) {
       const int q = qdiv(e, p.m_n0);
       const int x = e - q * p.N0;
       const long long pix = pix0 + e;
@@ -696,7 +725,7 @@ __device__ __forceinline__ void fft_forward_first_body(const FirstPass& p, int b
     for (int c = 0; c < ng; c++) {
       float2* dst = p.out + (long long)(c0 + c) * cout + (long long)l0 * p.G0;
 #pragma unroll 4
-      for (int e = threadIdx.x; e < per_coil; e += kFftThreads) {
+      for (int e = threadIdx.x; e < per_coil; e += NT) {
         const int q = qdiv(e, p.m_g0);
         const int x = e - q * p.G0;
         dst[e] = buf[(c * nq + q) * p.LP + x];
@@ -708,6 +737,16 @@ __device__ __forceinline__ void fft_forward_first_body(const FirstPass& p, int b
 template <bool PR>
 __global__ void __launch_bounds__(kFftThreads, 4) fft_adjoint_last_kernel(LastPass p) {
   fft_adjoint_last_body(p, blockIdx.x, RunTable<PR>{p.st, p.n_st});
+}
+
+template <int NT, bool PR>
+__global__ void __launch_bounds__(NT, PR ? 4 : 8) fft_adjoint_last_light_kernel(LastPass p) {
+  fft_adjoint_last_body(p, blockIdx.x, RunTable<PR, NT, kLightPerThread>{p.st, p.n_st});
+}
+
+template <int NT, bool PR>
+__global__ void __launch_bounds__(NT, PR ? 4 : 8) fft_forward_first_light_kernel(FirstPass p) {
+  fft_forward_first_body(p, blockIdx.x, RunTable<PR, NT, kLightPerThread>{p.st, p.n_st});
 }
 
 template <int L, int... R>
@@ -834,38 +873,6 @@ void x_tiling(int G0, int N0, int coils, int* Cg, int* Q) {
   *Q = std::max(1, std::min(per_tile / *Cg, (kMaxPix * kFftThreads) / N0));
 }
 
-// The stage table of axis a inside the device table buffer.
-const FftStage* stage_table(const float2* tw, const size_t tw_off[3][3], int a) {
-  return reinterpret_cast<const FftStage*>(tw + tw_off[a][2]);
-}
-
-// Tiling of a y / z pass (the caller fills the geometry fields).
-bool finish_axis(AxisPass* p, int coils, const FftStage* st) {
-  p->coils = coils;
-  p->LP = pad_of(p->L);
-  FftRadices r;
-  if (!make_radices(p->L, &r)) return false;
-  p->st = st;
-  p->n_st = r.n;
-  // 16-line tiles at least (128-byte rows): lines above 511 points take the
-  // large tile
-  p->big = 16 * p->LP > kTileElems ? 1 : 0;
-  const int tile = p->big ? kBigTileElems : kTileElems;
-  int lg = 0;
-  while ((2 << lg) <= kMaxStripe && (2 << lg) * p->LP <= tile) lg++;
-  p->stripe = 1 << lg;
-  p->m_stripe = qdiv_const(p->stripe);
-  p->x_tiles = (p->nx + p->stripe - 1) / p->stripe;
-  return true;
-}
-
-uint32_t axis_blocks(const AxisPass& p) { return (uint32_t)p.coils * p.nob * p.x_tiles; }
-size_t axis_lds(const AxisPass& p) { return tile_bytes(p.L, p.stripe); }
-uint32_t last_blocks(const LastPass& p) { return (uint32_t)((p.lines + p.Q - 1) / p.Q); }
-size_t last_lds(const LastPass& p) { return tile_bytes(p.G0, p.Q * p.Cg); }
-uint32_t first_blocks(const FirstPass& p) { return (uint32_t)((p.lines + p.Q - 1) / p.Q); }
-size_t first_lds(const FirstPass& p) { return tile_bytes(p.G0, p.Q * p.Cg); }
-
 // Line lengths with compile-time kernels: (L, tile lines of a y / z pass,
 // radices). The tile must be the one finish_axis picks for L. Besides the
 // common smooth lengths (and 320, the 160^3 osf-2 grid), the 3-D grids of
@@ -897,18 +904,97 @@ size_t first_lds(const FirstPass& p) { return tile_bytes(p.G0, p.Q * p.Cg); }
 #define GNUFFT_FIXED_X_SIZES(X) \
   X(512, 0, 8, 8, 8)
 
-template <typename K>
+// L has compile-time kernels (x: of an x pass).
+bool fixed_length(int L, bool x) {
+#define GNUFFT_LENGTH_CASE(LEN, TILE, ...) \
+  if (L == LEN) return true;
+  GNUFFT_FIXED_FFT_SIZES(GNUFFT_LENGTH_CASE)
+  if (x) {
+    GNUFFT_FIXED_X_SIZES(GNUFFT_LENGTH_CASE)
+  }
+#undef GNUFFT_LENGTH_CASE
+  return false;
+}
+
+// Threads of a light kernel for a tile of `elems` elements.
+int light_threads(int elems) {
+  int nt = 128;
+  while (nt * kLightPerThread < elems) nt *= 2;
+  return nt;
+}
+
+// Small transforms: fewer image lines per tile of an x pass until there are
+// tiles for two workgroups per CU; returns the light kernel's threads, or 0.
+int x_light(int G0, int lines, int Cg, int* Q) {
+  if (Cg * G0 > kLightPerThread * 1024) return 0;
+  if ((uint32_t)((lines + *Q - 1) / *Q) >= (fixed_length(G0, true) ? kLightFixed : kLightX)) return 0;
+  *Q = std::max(1, std::min(*Q, lines / 512));
+  return light_threads(Cg * *Q * G0);
+}
+
+// The stage table of axis a inside the device table buffer.
+const FftStage* stage_table(const float2* tw, const size_t tw_off[3][3], int a) {
+  return reinterpret_cast<const FftStage*>(tw + tw_off[a][2]);
+}
+
+// Tiling of a y / z pass (the caller fills the geometry fields).
+bool finish_axis(AxisPass* p, int coils, const FftStage* st, bool light) {
+  p->coils = coils;
+  p->LP = pad_of(p->L);
+  FftRadices r;
+  if (!make_radices(p->L, &r)) return false;
+  p->st = st;
+  p->n_st = r.n;
+  // 16-line tiles at least (128-byte rows): lines above 511 points take the
+  // large tile
+  p->big = 16 * p->LP > kTileElems ? 1 : 0;
+  const int tile = p->big ? kBigTileElems : kTileElems;
+  int lg = 0;
+  while ((2 << lg) <= kMaxStripe && (2 << lg) * p->LP <= tile) lg++;
+  p->stripe = 1 << lg;
+  p->x_tiles = (p->nx + p->stripe - 1) / p->stripe;
+  if (light && p->L <= kLightPerThread * 1024 / kLightStripe &&
+      (uint64_t)coils * p->nob * p->x_tiles < (fixed_length(p->L, false) ? kLightFixed : kLightBlocks)) {
+    p->stripe = kLightStripe;
+    p->light = light_threads(p->L * kLightStripe);
+    p->x_tiles = (p->nx + p->stripe - 1) / p->stripe;
+  }
+  p->m_stripe = qdiv_const(p->stripe);
+  return true;
+}
+
+uint32_t axis_blocks(const AxisPass& p) { return (uint32_t)p.coils * p.nob * p.x_tiles; }
+size_t axis_lds(const AxisPass& p) { return tile_bytes(p.L, p.stripe); }
+uint32_t last_blocks(const LastPass& p) { return (uint32_t)((p.lines + p.Q - 1) / p.Q); }
+size_t last_lds(const LastPass& p) { return tile_bytes(p.G0, p.Q * p.Cg); }
+uint32_t first_blocks(const FirstPass& p) { return (uint32_t)((p.lines + p.Q - 1) / p.Q); }
+size_t first_lds(const FirstPass& p) { return tile_bytes(p.G0, p.Q * p.Cg); }
+
+template <typename K, typename P>
 hipError_t launch_pass(K kernel, uint32_t blocks, size_t lds, hipStream_t s,
-                       const AxisPass& p, int threads = kFftThreads) {
+                       const P& p, int threads = kFftThreads) {
   hipError_t e = allow_lds(kernel, lds);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), lds, s, p);
   return hipGetLastError();
 }
 
+#define GNUFFT_LIGHT(KERNEL, PR, NT_)                     \
+  switch (NT_) {                                          \
+    case 128: GNUFFT_LIGHT_CASE(KERNEL, 128, PR)          \
+    case 256: GNUFFT_LIGHT_CASE(KERNEL, 256, PR)          \
+    case 512: GNUFFT_LIGHT_CASE(KERNEL, 512, PR)          \
+    default: GNUFFT_LIGHT_CASE(KERNEL, 1024, PR)          \
+  }
+#define GNUFFT_LIGHT_CASE(KERNEL, NT, PR) return launch_pass((KERNEL<NT, PR>), blocks, lds, s, p, NT);
+
 hipError_t launch_axis(const AxisPass& p, hipStream_t s) {
   const size_t lds = axis_lds(p);
   const uint32_t blocks = axis_blocks(p);
+  if (p.light) {
+    if (prime_radix(p.L)) GNUFFT_LIGHT(fft_axis_light_kernel, true, p.light)
+    GNUFFT_LIGHT(fft_axis_light_kernel, false, p.light)
+  }
 #define GNUFFT_AXIS_CASE(LEN, TILE, ...) \
   if (p.L == LEN && p.stripe == TILE)    \
     return launch_pass(fft_axis_fixed_kernel<LEN, TILE, __VA_ARGS__>, blocks, lds, s, p);
@@ -922,43 +1008,43 @@ hipError_t launch_axis(const AxisPass& p, hipStream_t s) {
   return launch_pass(fft_axis_kernel<false>, blocks, lds, s, p);
 }
 
-template <typename K, typename P>
-hipError_t launch_x(K kernel, uint32_t blocks, size_t lds, hipStream_t s, const P& p) {
-  hipError_t e = allow_lds(kernel, lds);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kFftThreads), lds, s, p);
-  return hipGetLastError();
-}
-
 hipError_t launch_last(const LastPass& p, hipStream_t s) {
   const size_t lds = last_lds(p);
   const uint32_t blocks = last_blocks(p);
+  if (p.light) {
+    if (prime_radix(p.G0)) GNUFFT_LIGHT(fft_adjoint_last_light_kernel, true, p.light)
+    GNUFFT_LIGHT(fft_adjoint_last_light_kernel, false, p.light)
+  }
 #define GNUFFT_LAST_CASE(LEN, TILE, ...) \
-  if (p.G0 == LEN) return launch_x(fft_adjoint_last_fixed_kernel<LEN, __VA_ARGS__>, blocks, lds, s, p);
+  if (p.G0 == LEN) return launch_pass(fft_adjoint_last_fixed_kernel<LEN, __VA_ARGS__>, blocks, lds, s, p);
   GNUFFT_FIXED_FFT_SIZES(GNUFFT_LAST_CASE)
   GNUFFT_FIXED_X_SIZES(GNUFFT_LAST_CASE)
 #undef GNUFFT_LAST_CASE
-  if (prime_radix(p.G0)) return launch_x(fft_adjoint_last_kernel<true>, blocks, lds, s, p);
-  return launch_x(fft_adjoint_last_kernel<false>, blocks, lds, s, p);
+  if (prime_radix(p.G0)) return launch_pass(fft_adjoint_last_kernel<true>, blocks, lds, s, p);
+  return launch_pass(fft_adjoint_last_kernel<false>, blocks, lds, s, p);
 }
 
 hipError_t launch_first(const FirstPass& p, hipStream_t s) {
   const size_t lds = first_lds(p);
   const uint32_t blocks = first_blocks(p);
+  if (p.light) {
+    if (prime_radix(p.G0)) GNUFFT_LIGHT(fft_forward_first_light_kernel, true, p.light)
+    GNUFFT_LIGHT(fft_forward_first_light_kernel, false, p.light)
+  }
 #define GNUFFT_FIRST_CASE(LEN, TILE, ...) \
-  if (p.G0 == LEN) return launch_x(fft_forward_first_fixed_kernel<LEN, __VA_ARGS__>, blocks, lds, s, p);
+  if (p.G0 == LEN) return launch_pass(fft_forward_first_fixed_kernel<LEN, __VA_ARGS__>, blocks, lds, s, p);
   GNUFFT_FIXED_FFT_SIZES(GNUFFT_FIRST_CASE)
   GNUFFT_FIXED_X_SIZES(GNUFFT_FIRST_CASE)
 #undef GNUFFT_FIRST_CASE
-  if (prime_radix(p.G0)) return launch_x(fft_forward_first_kernel<true>, blocks, lds, s, p);
-  return launch_x(fft_forward_first_kernel<false>, blocks, lds, s, p);
+  if (prime_radix(p.G0)) return launch_pass(fft_forward_first_kernel<true>, blocks, lds, s, p);
+  return launch_pass(fft_forward_first_kernel<false>, blocks, lds, s, p);
 }
 
 // Pass descriptors of the adjoint: grid [coils][G2][G1][G0] (the
 // INVERSE-shifted spectrum) -> image; ax[0 .. d-2] then the x pass.
 bool build_adjoint(const Geom& g, float2* grid, float2* tmp, int coils, const float* deapo,
                    const float2* sens, float2* out, int stop, bool accumulate, const float2* tw,
-                   const size_t tw_off[3][3], AxisPass ax[2], LastPass* last) {
+                   const size_t tw_off[3][3], AxisPass ax[2], LastPass* last, bool light) {
   const float sign = 1.0f;  // unnormalised inverse transform
   const int G0 = g.G[0], G1 = g.G[1];
   const int N1 = g.N[1], N2 = g.dim == 3 ? g.N[2] : 1;
@@ -983,7 +1069,7 @@ bool build_adjoint(const Geom& g, float2* grid, float2* tmp, int coils, const fl
     z.out_off = g.crop[2] + g.shift_inv[2];
     z.sign = sign;
     z.tw = tw + tw_off[2][1];
-    if (!finish_axis(&z, coils, stage_table(tw, tw_off, 2))) return false;
+    if (!finish_axis(&z, coils, stage_table(tw, tw_off, 2), light)) return false;
     cur = tmp;
   }
   // y: [c][N2][G1][G0] -> [c][N2][N1][G0] (3-D: tmp -> grid, 2-D: grid -> tmp)
@@ -1006,7 +1092,7 @@ bool build_adjoint(const Geom& g, float2* grid, float2* tmp, int coils, const fl
   y.out_off = g.crop[1] + g.shift_inv[1];
   y.sign = sign;
   y.tw = tw + tw_off[1][1];
-  if (!finish_axis(&y, coils, stage_table(tw, tw_off, 1))) return false;
+  if (!finish_axis(&y, coils, stage_table(tw, tw_off, 1), light)) return false;
   LastPass& p = *last;
   p = LastPass{};
   p.in = ydst;
@@ -1021,6 +1107,7 @@ bool build_adjoint(const Geom& g, float2* grid, float2* tmp, int coils, const fl
   p.shift0 = g.shift_inv[0];
   p.coils = coils;
   x_tiling(G0, p.N0, coils, &p.Cg, &p.Q);
+  if (light) p.light = x_light(G0, p.lines, p.Cg, &p.Q);
   p.m_g0 = qdiv_const(G0);
   p.m_n0 = qdiv_const(p.N0);
   p.scale = g.fft_scale;
@@ -1039,7 +1126,7 @@ bool build_adjoint(const Geom& g, float2* grid, float2* tmp, int coils, const fl
 // pass, then ax[0 .. d-2] (y, z).
 bool build_forward(const Geom& g, const float2* img, bool img_per_coil, const float2* sens,
                    const float* deapo, float2* grid, float2* tmp, int coils, const float2* tw,
-                   const size_t tw_off[3][3], FirstPass* first, AxisPass ax[2]) {
+                   const size_t tw_off[3][3], FirstPass* first, AxisPass ax[2], bool light) {
   const float sign = -1.0f;
   const int G0 = g.G[0], G1 = g.G[1];
   const int N1 = g.N[1], N2 = g.dim == 3 ? g.N[2] : 1;
@@ -1057,6 +1144,7 @@ bool build_forward(const Geom& g, const float2* img, bool img_per_coil, const fl
   f.shift0 = g.shift_inv[0];
   f.coils = coils;
   x_tiling(G0, f.N0, coils, &f.Cg, &f.Q);
+  if (light) f.light = x_light(G0, f.lines, f.Cg, &f.Q);
   f.m_g0 = qdiv_const(G0);
   f.m_n0 = qdiv_const(f.N0);
   f.m_pad = G0 > f.N0 ? qdiv_const(G0 - f.N0) : 0;
@@ -1088,7 +1176,7 @@ bool build_forward(const Geom& g, const float2* img, bool img_per_coil, const fl
   y.in_off = g.crop[1] - g.shift_inv[1];
   y.sign = sign;
   y.tw = tw + tw_off[1][0];
-  if (!finish_axis(&y, coils, stage_table(tw, tw_off, 1))) return false;
+  if (!finish_axis(&y, coils, stage_table(tw, tw_off, 1), light)) return false;
   if (g.dim == 2) return true;
   // z: [c][N2][G1][G0] -> [c][G2][G1][G0]
   AxisPass& z = ax[1];
@@ -1108,7 +1196,7 @@ bool build_forward(const Geom& g, const float2* img, bool img_per_coil, const fl
   z.in_off = g.crop[2] - g.shift_inv[2];
   z.sign = sign;
   z.tw = tw + tw_off[2][0];
-  return finish_axis(&z, coils, stage_table(tw, tw_off, 2));
+  return finish_axis(&z, coils, stage_table(tw, tw_off, 2), light);
 }
 
 }  // namespace
@@ -1184,7 +1272,7 @@ hipError_t fused_fft_adjoint(const Geom& g, float2* grid, float2* tmp, int coils
   AxisPass ax[2];
   LastPass last;
   if (!build_adjoint(g, grid, tmp, coils, deapo, sens, out, stop, accumulate, tw, tw_off, ax,
-                     &last))
+                     &last, true))
     return hipErrorInvalidValue;
   for (int i = 0; i < g.dim - 1; i++) {
     hipError_t e = launch_axis(ax[i], s);
@@ -1202,7 +1290,7 @@ hipError_t fused_fft_forward(const Geom& g, const float2* img, bool img_per_coil
                              hipStream_t s) {
   FirstPass first;
   AxisPass ax[2];
-  if (!build_forward(g, img, img_per_coil, sens, deapo, grid, tmp, coils, tw, tw_off, &first, ax))
+  if (!build_forward(g, img, img_per_coil, sens, deapo, grid, tmp, coils, tw, tw_off, &first, ax, true))
     return hipErrorInvalidValue;
   hipError_t e = launch_first(first, s);
   for (int i = 0; i < g.dim - 1 && e == hipSuccess; i++) e = launch_axis(ax[i], s);
@@ -1223,9 +1311,9 @@ bool fused_fft_desc_build(void* desc, const Geom& g, float2* grid, float2* tmp, 
   d = FftOpDesc{};
   d.n_ax = g.dim - 1;
   return build_adjoint(g, grid, tmp, coils, deapo, sens, nullptr, 2, false, tw, tw_off, d.adj_ax,
-                       &d.adj_x) &&
+                       &d.adj_x, false) &&
          build_forward(g, nullptr, sens == nullptr, sens, deapo, grid, tmp, coils, tw, tw_off,
-                       &d.fwd_x, d.fwd_ax);
+                       &d.fwd_x, d.fwd_ax, false);
 }
 
 void fused_fft_desc_set_io(void* desc, float2* adjoint_out, const float2* forward_img) {
