@@ -195,22 +195,23 @@ __device__ __forceinline__ void tile_spread_body(const Geom& g, const SpreadArgs
   float sq[S::VI];
   float4 v[S::VI];
   uint32_t je = 0, jv[S::VI];  // list words of the round after the loaded one
-  auto load_words = [&](uint64_t r0) {
-    if (has_axis && r0 + e < n) je = entries[r0 + e];
+  const uint32_t rounds = (n + ER - 1) / ER;
+  auto at = [&](uint32_t r, int k) { return r * ER + (uint32_t)k; };  // list position of sample k of round r
+  auto load_words = [&](uint32_t r) {
+    if (has_axis && at(r, e) < n) je = entries[at(r, e)];
 #pragma unroll
     for (int q = 0; q < S::VI; q++) {
-      const uint64_t at = r0 + ve + q * (S::NT / S::PP);
-      if (has_value && at < n) jv[q] = entries[at];
+      const int k = ve + q * (S::NT / S::PP);
+      if (has_value && at(r, k) < n) jv[q] = entries[at(r, k)];
     }
   };
-  auto load_round = [&](uint64_t r0) {
-    if (has_axis && r0 + e < n) ta = load_taps<NX>(taps + (size_t)je * (NX / 4));
+  auto load_round = [&](uint32_t r) {
+    if (has_axis && at(r, e) < n) ta = load_taps<NX>(taps + (size_t)je * (NX / 4));
 #pragma unroll
     for (int q = 0; q < S::VI; q++) {
-      const uint64_t at = r0 + ve + q * (S::NT / S::PP);
       v[q] = make_float4(0.f, 0.f, 0.f, 0.f);
       sq[q] = 1.0f;
-      if (!has_value || at >= n) continue;
+      if (!has_value || at(r, ve + q * (S::NT / S::PP)) >= n) continue;
       if (dens) sq[q] = a.dens[jv[q]];
       if (coils > 0) {
         const float2 t = data[jv[q]];
@@ -224,7 +225,7 @@ __device__ __forceinline__ void tile_spread_body(const Geom& g, const SpreadArgs
   };
   load_words(0);
   load_round(0);
-  load_words(ER);
+  load_words(1);
   if (tid < ST) ent[ER * ST + tid] = 0.0f;  // the padding sample
 
   // sub-tile of this wave
@@ -242,10 +243,11 @@ __device__ __forceinline__ void tile_spread_body(const Geom& g, const SpreadArgs
   const int off_x = S::SX * sx + xi;
   const int off_v = S::SUM + vi;
 
-  for (uint32_t r0 = 0; r0 < n; r0 += ER) {
-    const int rn = (int)min((uint32_t)ER, n - r0);
-    // stage this round's samples
-    if (has_axis && e < rn) {
+  for (uint32_t round = 0; round < rounds; round++) {
+    // stage this round's samples (no hits where the list has ended)
+    if (has_axis && at(round, e) >= n) {
+      hit[4 * e + axis] = 0;
+    } else if (has_axis) {
       const int T = axis == 0 ? S::TX : axis == 1 ? S::TY : S::TZ;
       const int before = axis == 0 ? 0 : axis == 1 ? S::TX : S::TX + S::TY;
       hit[4 * e + axis] = (uint8_t)tile_weights<NX>(ta, t0[axis], T, g.G[axis], ent + e * ST + before);
@@ -253,14 +255,14 @@ __device__ __forceinline__ void tile_spread_body(const Geom& g, const SpreadArgs
 #pragma unroll
     for (int q = 0; q < S::VI; q++) {
       const int s = ve + q * (S::NT / S::PP);
-      if (!has_value || s >= rn) continue;
+      if (!has_value || at(round, s) >= n) continue;
       float2* to = reinterpret_cast<float2*>(ent + s * ST + S::SUM + 4 * part);
       to[0] = make_float2(v[q].x * sq[q], v[q].y * sq[q]);
       to[1] = make_float2(v[q].z * sq[q], v[q].w * sq[q]);
     }
     __syncthreads();
-    load_round((uint64_t)r0 + ER);
-    load_words((uint64_t)r0 + 2 * ER);
+    load_round(round + 1);
+    load_words(round + 2);
 
     // this wave's samples of the round: rank q sits at [q % 4][q / 4], the
     // order in which lane group q % 4 consumes them, padded to whole pairs
@@ -269,12 +271,9 @@ __device__ __forceinline__ void tile_spread_body(const Geom& g, const SpreadArgs
 #pragma unroll
     for (int q = 0; q < ER / 64; q++) {
       const int s = q * 64 + lane;
-      bool in = false;
-      if (s < rn) {
-        const uint32_t hb = *reinterpret_cast<const uint32_t*>(hit + 4 * s);
-        in = (hb >> sx) & 1u;
-        if (DIM == 3) in = in && ((hb >> (8 + sy)) & 1u);
-      }
+      const uint32_t hb = *reinterpret_cast<const uint32_t*>(hit + 4 * s);
+      bool in = (hb >> sx) & 1u;
+      if (DIM == 3) in = in && ((hb >> (8 + sy)) & 1u);
       const uint64_t b = __ballot(in);
       if (in) {
         const int rank = cnt + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32),
@@ -360,8 +359,11 @@ __device__ __forceinline__ void tile_spread_body(const Geom& g, const SpreadArgs
   }
 }
 
+// Four workgroups of 8 waves fill a CU up to 64 registers (two more cost 15 us
+// of 683 at 128^3).
 template <int DIM, int NC, int NX>
-__global__ void __launch_bounds__((TileShape<DIM, NC>::NT)) tile_spread_kernel(Geom g, SpreadArgs a) {
+__global__ void __launch_bounds__((TileShape<DIM, NC>::NT))
+    __attribute__((amdgpu_waves_per_eu(DIM == 3 && NX == 4 ? 8 : 4))) tile_spread_kernel(Geom g, SpreadArgs a) {
   const uint32_t ci = run_item(blockIdx.x);
   if (ci >= a.tiles.n_chunks) return;
   tile_spread_body<DIM, NC, NX>(g, a, ci, blockIdx.y);
