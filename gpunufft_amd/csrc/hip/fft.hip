@@ -57,6 +57,11 @@ constexpr int kBigTileElems = kPerThread * kBigThreads;
 // (constant strides) keep them down to one tile per CU: x passes of 512 points
 // take 18 and 16 us, light ones 21 and 18.
 constexpr int kLightPerThread = 8;
+// y / z passes of short lines without kernels of their own (32 lines of up to 128
+// points): half the threads, since a prime stage has a butterfly for few of 512
+// (192 of them at 66 = 2 * 3 * 11 points) and a CU holds twice as many such tiles.
+// 252 x 240 x 66, 6 coils: 135 -> 94 us a pass (0.32 GB, 67 us at 4.8 TB/s).
+constexpr int kShortThreads = 256;
 constexpr int kLightStripe = 8;
 constexpr uint32_t kLightBlocks = 2048, kLightX = 512;  // tiles of a y / z and of an x pass
 constexpr uint32_t kLightFixed = 256;                   // line lengths with kernels of their own
@@ -416,6 +421,7 @@ struct AxisPass {
   int stripe, x_tiles, coils;
   int big;  // 1: lines above 511 points, kBigThreads and a kBigTileElems tile
   int light;  // threads of the light kernel, 0: not used
+  int short_lines;  // 1: kShortThreads are enough for the tile
   uint32_t m_stripe;
   float sign;
   const FftStage* st;  // stage table in device memory (beside the twiddles)
@@ -481,6 +487,11 @@ __global__ void __launch_bounds__(kFftThreads, 4) fft_axis_kernel(AxisPass p) {
 template <bool PR>
 __global__ void __launch_bounds__(kBigThreads, 1) fft_axis_big_kernel(AxisPass p) {
   fft_axis_body<kBigThreads, PR>(p, blockIdx.x);
+}
+
+template <bool PR>
+__global__ void __launch_bounds__(kShortThreads, 4) fft_axis_short_kernel(AxisPass p) {
+  fft_axis_body<kShortThreads, PR>(p, blockIdx.x);
 }
 
 template <int NT, bool PR>
@@ -959,6 +970,7 @@ bool finish_axis(AxisPass* p, int coils, const FftStage* st, bool light) {
     p->light = light_threads(p->L * kLightStripe);
     p->x_tiles = (p->nx + p->stripe - 1) / p->stripe;
   }
+  p->short_lines = light && !p->light && p->L * p->stripe <= kPerThread * kShortThreads ? 1 : 0;
   p->m_stripe = qdiv_const(p->stripe);
   return true;
 }
@@ -1000,6 +1012,10 @@ hipError_t launch_axis(const AxisPass& p, hipStream_t s) {
     return launch_pass(fft_axis_fixed_kernel<LEN, TILE, __VA_ARGS__>, blocks, lds, s, p);
   GNUFFT_FIXED_FFT_SIZES(GNUFFT_AXIS_CASE)
 #undef GNUFFT_AXIS_CASE
+  if (p.short_lines) {
+    if (prime_radix(p.L)) return launch_pass(fft_axis_short_kernel<true>, blocks, lds, s, p, kShortThreads);
+    return launch_pass(fft_axis_short_kernel<false>, blocks, lds, s, p, kShortThreads);
+  }
   if (prime_radix(p.L)) {
     if (p.big) return launch_pass(fft_axis_big_kernel<true>, blocks, lds, s, p, kBigThreads);
     return launch_pass(fft_axis_kernel<true>, blocks, lds, s, p);

@@ -1,6 +1,8 @@
-"""FFT passes of small grids (few tiles) at the edges of their tiles: the light
-kernels run the same stages in the same order as the full tiles that a batch
-uses, so a plan by itself and a batch of that plan give the same bits.
+"""FFT passes of small grids (few tiles) and of short lines at the edges of their
+tiles: the light and the short-line kernels run the same stages in the same
+order as the full tiles that a batch uses, so a plan by itself and a batch of
+that plan give the same bits (for lengths without kernels of their own, which a
+batch does not use).
 """
 
 import numpy as np
@@ -25,6 +27,10 @@ CASES = [
     ((143, 152), 1.0, 5, True),
     ((480, 450), 2.0, 9, True),
     ((24, 20, 18), 1.5, 2, True),
+    # short lines with many tiles: 66 points in y, 22 and 4 in z
+    ((100, 44, 176), 1.5, 3, True),
+    ((165, 110, 22), 1.0, 8, False),
+    ((165, 100, 4), 1.0, 12, True),
 ]
 
 
