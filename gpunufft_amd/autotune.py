@@ -1,10 +1,10 @@
 """Sector-width autotuner.
 
-The sector width trades LDS footprint and per-sector fixed costs (staging,
-sub-grid stores, fold) against sector occupancy. The best width depends on
+The sector width trades LDS footprint and per-sector fixed costs (the
+interp's staging) against sector occupancy. The best width depends on
 the image size, trajectory density and coil count. For one operator
 shape, best_sector_width builds a plan for every candidate width, times the
-spread (with its reduction and fold) and the interpolation on device-resident
+spread (with its reduction) and the interpolation on device-resident
 data with HIP events, and returns the fastest width. Results are cached per
 (image size, kernel width, osf, sample count, coil count) so operators of one
 shape are tuned once.

@@ -1967,7 +1967,7 @@ int gnufft_batch_forward(gnufft_batch b, const void* const* img, void* const* ou
 
 // ---------------------------------------------------------------------------
 // Adjoint without allocation (no counterpart in the reference): the work
-// grid and the spread sub-grids live in a fixed per-device area, so the call
+// grid and the spread's partial tiles live in a fixed per-device area, so the call
 // makes no hipMalloc / hipFree and no allocating library call. The area is
 // a file-scope device array; host code uses only the address that
 // hipGetSymbolAddress returns for the current device (the array's host-side
@@ -2024,7 +2024,7 @@ int gnufft_adjoint_noalloc(gnufft_plan p, const void* kdata, void* out, uint32_t
                 "adjoint_noalloc: needs the fused FFT (rocFFT plans allocate work memory)");
   const Geom& g = p->g;
   // per coil: work grid (unless the caller's buffer is the grid) and the
-  // spread sub-grids / fused FFT intermediate
+  // partial tiles / fused FFT intermediate
   const size_t grid_b = grid_out ? 0 : (size_t)g.Ng * sizeof(float2);
   const size_t scr_b = scratch_bytes(p, 1);
   const size_t per = round_up_256(grid_b) + round_up_256(scr_b);

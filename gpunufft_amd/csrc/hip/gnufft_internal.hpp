@@ -346,10 +346,10 @@ __device__ __host__ inline uint32_t tile_chunk(int dim, uint64_t pairs) {
 
 // gridding.hip
 
-// Chunks per interp run: 4 stages the dense k-space centre's sectors fewer
-// times at the 128^3 koosh workload (interp 0.62 -> 0.60 ms); 8 and whole
-// sectors leave a long tail of busy workgroups (0.67 and 1.62 ms).
-constexpr int kInterpRun = 4;
+// Chunks per 3-D interp run, which stages its sector once. Interp at 128^3 koosh /
+// a 168 x 160 x 44 stack / 160^3: 459 / 140 / 759 us with 1, 450 / 143 / 757 with 2,
+// 449 / 152 / 760 with 4, 469 / 155 / 754 with 8 (a tail of busy workgroups).
+constexpr int kInterpRun = 2;
 
 // Gridding work list: chunks in sector order, split into 8 contiguous
 // ranges of about equal cost; range x is processed on XCD x (workgroups

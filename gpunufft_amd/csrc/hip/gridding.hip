@@ -29,7 +29,9 @@
 // 2.0 M samples, 8 coils), 0.30 -> 0.15 ms (168 x 160 x 44 stack, 6 coils),
 // 66 -> 26 us (256^2 osf 2, 16 coils), 143 -> 17 us (224^2 kernel width 5,
 // 12 coils), 5.3 -> 4.4 us (64^2, 1 coil).
-// Two staging loads more in flight take 90 registers: 26 -> 30 us at 256^2.
+// Eight staging loads in flight instead of four take 90 registers: 26 -> 30 us at
+// 256^2.
+
 #include <algorithm>
 #include <type_traits>
 
@@ -66,8 +68,8 @@ static void split_ranges(const uint32_t* costs, uint32_t n, uint32_t begin[9], u
 }
 
 void partition_work(const uint32_t* counts, uint32_t n, WorkList* w) {
-  // Cost of a chunk: its samples plus a fixed share for staging and
-  // storing the padded sub-grid (about 300 samples' worth on gfx950).
+  // Cost of a chunk: its samples plus a fixed share for staging the padded
+  // sector (about 300 samples' worth on gfx950).
   std::vector<uint32_t> cost(n);
   for (uint32_t i = 0; i < n; i++) cost[i] = counts[i] + 300u;
   split_ranges(cost.data(), n, w->xcd_begin, &w->max_range);

@@ -36,9 +36,9 @@
 // workgroup waiting for the one with the most samples of a round (half of the
 // wave cycles; matrix cores busy 30 %).
 // Spread and fold, measured against sector sub-grids in LDS with a fold over
-// neighbouring sectors: 0.91 -> 0.77 ms (128^3 koosh, 8 coils), 2.52 -> 0.80 ms
-// (160^3 osf 2, 2.0 M samples, 8 coils), 0.59 -> 0.27 ms (168 x 160 x 44 stack,
-// 6 coils), 126 -> 49 us (256^2 osf 2, 16 coils), 123 -> 33 us (224^2 kernel
+// neighbouring sectors: 0.91 -> 0.68 ms (128^3 koosh, 8 coils), 2.52 -> 0.81 ms
+// (160^3 osf 2, 2.0 M samples, 8 coils), 0.59 -> 0.25 ms (168 x 160 x 44 stack,
+// 6 coils), 126 -> 46 us (256^2 osf 2, 16 coils), 123 -> 32 us (224^2 kernel
 // width 5, 12 coils), 13 -> 10 us (64^2, 1 coil).
 
 #include <algorithm>

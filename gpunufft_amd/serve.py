@@ -63,8 +63,8 @@ class Request:
         M = self.traj.shape[1]
         C = self.coils
         P = self.sector_width + 2 * (self.kernel_width // 2)
-        # grid + FFT work, sub-grid scratch (chunks ~ sectors), sens, data,
-        # CG vectors, tables
+        # grid + FFT work, gridding scratch and tap tables (bounded by padded
+        # sectors), sens, data, CG vectors, tables
         sectors = int(np.prod([math.ceil(int(n * self.osf) / self.sector_width)
                                for n in self.img_dims]))
         scratch = (sectors + M // 1024 + 1) * C * P ** d * 8
