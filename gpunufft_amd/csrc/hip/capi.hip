@@ -260,6 +260,16 @@ struct gnufft_plan_s {
   TileTask* tile_tasks_d = nullptr;
   TileList tiles{};
   uint32_t n_slots = 0;
+  // sector sums (CG-SENSE on odd grids; built by the first solve): chunks, the
+  // sectors' first chunks, per axis the sectors covering a grid index (kept with
+  // the plan), sub-grids
+  Chunk* sums_chunks_d = nullptr;
+  uint32_t* sums_first_d = nullptr;
+  uint32_t n_sums_chunks = 0;
+  uint32_t* cover_off_d[3] = {nullptr, nullptr, nullptr};
+  uint2* cover_d[3] = {nullptr, nullptr, nullptr};
+  float2* sub_d = nullptr;
+  size_t sub_cap = 0;  // bytes
   // partial tiles [slot][coil][tile point], or the fused FFT's intermediate;
   // capacity in bytes
   float2* scratch_d = nullptr;
@@ -303,6 +313,12 @@ struct gnufft_plan_s {
 
 uint64_t gnufft::plan_generation(const gnufft_plan_s* p) { return p ? p->generation : 0; }
 
+bool gnufft::plan_odd_grid(const gnufft_plan_s* p) {
+  for (int a = 0; a < p->g.dim; a++)
+    if (p->g.G[a] % 2) return true;
+  return false;
+}
+
 namespace {
 
 void dfree(void* p) {
@@ -327,6 +343,14 @@ void free_traj(gnufft_plan p) {
   dfree(p->tile_entries_d);
   dfree(p->tile_chunks_d);
   dfree(p->tile_tasks_d);
+  dfree(p->sums_chunks_d);
+  dfree(p->sums_first_d);
+  dfree(p->sub_d);
+  p->sums_chunks_d = nullptr;
+  p->sums_first_d = nullptr;
+  p->n_sums_chunks = 0;
+  p->sub_d = nullptr;
+  p->sub_cap = 0;
   p->traj_sorted_d = p->dens_sorted_d = nullptr;
   p->idx_d = p->assigned_d = p->sdc_d = p->centers_d = nullptr;
   p->chunks_d = nullptr;
@@ -485,14 +509,16 @@ int ensure_scratch_bytes(gnufft_plan p, size_t bytes) {
 
 int ensure_scratch(gnufft_plan p, uint32_t coils) { return ensure_scratch_bytes(p, scratch_bytes(p, coils)); }
 
-uint32_t coil_batch(gnufft_plan p, uint32_t n_coils) {
+// sub: bytes per coil of the sector sums' sub-grids, where they are used
+uint32_t coil_batch(gnufft_plan p, uint32_t n_coils, size_t sub = 0) {
   // buffers already hold every coil (steady state, e.g. under graph capture)
-  if (p->grid_coils >= n_coils && p->scratch_cap >= scratch_bytes(p, n_coils)) return n_coils;
+  if (p->grid_coils >= n_coils && p->scratch_cap >= scratch_bytes(p, n_coils) && p->sub_cap >= sub * n_coils)
+    return n_coils;
   size_t fr = 0, tot = 0;
   if (hipMemGetInfo(&fr, &tot) != hipSuccess) return 1;
   // grid + FFT work + scratch
-  size_t per = (size_t)p->g.Ng * sizeof(float2) * 2 + (scratch_bytes(p, 8) + 7) / 8;
-  size_t avail = fr / 2 + (size_t)p->grid_coils * p->g.Ng * sizeof(float2) + p->scratch_cap;
+  size_t per = (size_t)p->g.Ng * sizeof(float2) * 2 + (scratch_bytes(p, 8) + 7) / 8 + sub;
+  size_t avail = fr / 2 + (size_t)p->grid_coils * p->g.Ng * sizeof(float2) + p->scratch_cap + (sub ? p->sub_cap : 0);
   size_t cc = per ? avail / per : n_coils;
   if (cc < 1) cc = 1;
   return (uint32_t)std::min<size_t>(cc, n_coils);
@@ -812,6 +838,72 @@ int build_short(gnufft_plan p, const float* traj, uint32_t M, const float* dens,
   return GNUFFT_OK;
 }
 
+// Tables of the sector sums, unless they are there.
+int ensure_sums(gnufft_plan p, hipStream_t s) {
+  const Geom& g = p->g;
+  for (int a = 0; a < g.dim; a++) {
+    if (p->cover_d[a]) continue;
+    std::vector<uint32_t> off;
+    std::vector<uint2> entries;
+    sector_cover(g, a, &off, &entries);
+    int rc = copy_in((void**)&p->cover_off_d[a], off.data(), off.size() * sizeof(uint32_t), GNUFFT_HOST, s);
+    if (rc == GNUFFT_OK)
+      rc = copy_in((void**)&p->cover_d[a], entries.data(), entries.size() * sizeof(uint2), GNUFFT_HOST, s);
+    const hipError_t waited = hipStreamSynchronize(s);  // copies from locals
+    if (rc == GNUFFT_OK && waited != hipSuccess) rc = fail(GNUFFT_ERR_DEVICE, "sector sums: tables");
+    if (rc != GNUFFT_OK) {
+      dfree(p->cover_off_d[a]);
+      dfree(p->cover_d[a]);
+      p->cover_off_d[a] = nullptr;
+      p->cover_d[a] = nullptr;
+      return rc;
+    }
+  }
+  if (p->sums_first_d) return GNUFFT_OK;
+  std::vector<uint32_t> sdc((size_t)p->S + 1), first;
+  HIP_TRY(hipMemcpyAsync(sdc.data(), p->sdc_d, sdc.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipStreamSynchronize(s));
+  std::vector<Chunk> chunks;
+  for (uint32_t i = 0; i < p->S; i++) {
+    first.push_back((uint32_t)chunks.size());
+    for (uint32_t b = sdc[i]; b < sdc[i + 1]; b += std::min(sdc[i + 1] - b, kSumsChunk))
+      chunks.push_back(Chunk{i, b, b + std::min(sdc[i + 1] - b, kSumsChunk), 0});
+  }
+  first.push_back((uint32_t)chunks.size());
+  int rc = GNUFFT_OK;
+  if (!chunks.empty())
+    rc = copy_in((void**)&p->sums_chunks_d, chunks.data(), chunks.size() * sizeof(Chunk), GNUFFT_HOST, s);
+  if (rc == GNUFFT_OK)
+    rc = copy_in((void**)&p->sums_first_d, first.data(), first.size() * sizeof(uint32_t), GNUFFT_HOST, s);
+  const hipError_t waited = hipStreamSynchronize(s);
+  if (rc == GNUFFT_OK && waited != hipSuccess) rc = fail(GNUFFT_ERR_DEVICE, "sector sums: tables");
+  if (rc != GNUFFT_OK) {
+    dfree(p->sums_chunks_d);
+    dfree(p->sums_first_d);
+    p->sums_chunks_d = nullptr;
+    p->sums_first_d = nullptr;
+    return rc;
+  }
+  p->n_sums_chunks = (uint32_t)chunks.size();
+  return GNUFFT_OK;
+}
+
+// Bytes per coil of the sector sums' sub-grids.
+size_t sub_bytes(gnufft_plan p) { return (size_t)p->n_sums_chunks * sector_sub_elems(p->g) * sizeof(float2); }
+
+int ensure_sub(gnufft_plan p, uint32_t coils) {
+  const size_t bytes = sub_bytes(p) * coils;
+  if (p->sub_cap >= bytes) return GNUFFT_OK;
+  p->generation++;
+  dfree(p->sub_d);
+  p->sub_d = nullptr;
+  p->sub_cap = 0;
+  if (hipMalloc(&p->sub_d, bytes) != hipSuccess)
+    return fail(GNUFFT_ERR_OUT_OF_MEMORY, "sector sums: sub-grid allocation");
+  p->sub_cap = bytes;
+  return GNUFFT_OK;
+}
+
 bool valid_stop(int stop) { return stop >= 0 && stop <= 3; }
 
 // Spread arguments shared by every entry point (no density).
@@ -844,6 +936,26 @@ hipError_t plan_spread(gnufft_plan p, const SpreadArgs& a, hipStream_t s) {
   if (a.n_coils == 0) return hipSuccess;
   if (!p->cover_ok || (p->n_chunks > 0 && !spread_supported(p->g))) return hipErrorInvalidValue;
   return launch_spread(p->g, a, s);
+}
+
+// The same with the sector sums.
+hipError_t plan_sector_spread(gnufft_plan p, const SpreadArgs& a, hipStream_t s) {
+  if (!p->cover_ok || (p->n_chunks > 0 && !spread_supported(p->g))) return hipErrorInvalidValue;
+  SectorSpreadArgs b{};
+  b.data = a.data;
+  b.coil_stride = a.coil_stride;
+  b.dens = a.dens;
+  b.taps = a.taps;
+  b.idx = p->idx_d;
+  b.chunks = p->sums_chunks_d;
+  b.first = p->sums_first_d;
+  for (int d = 0; d < p->g.dim; d++) b.cover_off[d] = p->cover_off_d[d], b.cover[d] = p->cover_d[d];
+  b.sub = p->sub_d;
+  b.grid = a.grid;
+  b.n_chunks = p->n_sums_chunks;
+  b.n_coils = a.n_coils;
+  b.fold_shift = a.fold_shift;
+  return launch_sector_spread(p->g, b, p->lane_per_cu, s);
 }
 
 }  // namespace
@@ -1067,6 +1179,10 @@ int gnufft_plan_destroy(gnufft_plan p) {
   dfree(p->scratch_d);
   dfree(p->short_d);
   if (p->short_host) (void)hipHostFree(p->short_host);
+  for (int a = 0; a < 3; a++) {
+    dfree(p->cover_off_d[a]);
+    dfree(p->cover_d[a]);
+  }
   dfree(p->lut_d);
   dfree(p->deapo_d);
   dfree(p->sens_d);
@@ -1418,6 +1534,13 @@ int gnufft_interp_sorted(gnufft_plan p, const void* grid, void* data_sorted, uin
 
 int gnufft_adjoint(gnufft_plan p, const void* kdata, void* out, uint32_t n_coils, int stop,
                    void* stream) {
+  return plan_adjoint(p, kdata, out, n_coils, stop, false, stream);
+}
+
+}  // extern "C"
+
+int gnufft::plan_adjoint(gnufft_plan_s* p, const void* kdata, void* out, uint32_t n_coils, int stop, bool sector_sums,
+                         void* stream) {
   if (!p || !out || (!kdata && p->M)) return fail(GNUFFT_ERR_INVALID_ARGUMENT, "adjoint: null argument");
   if (!valid_stop(stop)) return fail(GNUFFT_ERR_INVALID_ARGUMENT, "adjoint: unknown stop stage");
   if (!p->sdc_d) return fail(GNUFFT_ERR_STATE, "adjoint: no trajectory set");
@@ -1428,13 +1551,18 @@ int gnufft_adjoint(gnufft_plan p, const void* kdata, void* out, uint32_t n_coils
   hipStream_t s = (hipStream_t)stream;
   const Geom& g = p->g;
   const bool grid_out = stop == GNUFFT_STOP_CONVOLUTION || stop == GNUFFT_STOP_DENSITY_ESTIMATION;
-  const uint32_t cc = coil_batch(p, n_coils);
+  if (sector_sums) {
+    int rc = ensure_sums(p, s);
+    if (rc) return rc;
+  }
+  const uint32_t cc = coil_batch(p, n_coils, sector_sums ? sub_bytes(p) : 0);
   if (!grid_out) {
     int rc = ensure_grid(p, cc);
     if (rc) return rc;
   }
   {
     int rc = ensure_scratch(p, cc);
+    if (rc == GNUFFT_OK && sector_sums) rc = ensure_sub(p, cc);
     if (rc) return rc;
   }
   for (uint32_t c0 = 0; c0 < n_coils; c0 += cc) {
@@ -1444,7 +1572,7 @@ int gnufft_adjoint(gnufft_plan p, const void* kdata, void* out, uint32_t n_coils
       SpreadArgs a = spread_args(p, (const float2*)kdata + (size_t)c0 * p->M, grid, nc);
       a.dens = p->dens_sqrt_d;
       a.fold_shift = !grid_out;
-      TIMED(p, GNUFFT_T_SPREAD, s, plan_spread(p, a, s));
+      TIMED(p, GNUFFT_T_SPREAD, s, sector_sums ? plan_sector_spread(p, a, s) : plan_spread(p, a, s));
     }
     if (grid_out) continue;
     if (p->fused) {
@@ -1467,6 +1595,8 @@ int gnufft_adjoint(gnufft_plan p, const void* kdata, void* out, uint32_t n_coils
   }
   return GNUFFT_OK;
 }
+
+extern "C" {
 
 int gnufft_forward(gnufft_plan p, const void* img, void* out, uint32_t n_coils, int stop,
                    void* stream) {

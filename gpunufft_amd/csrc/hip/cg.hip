@@ -180,10 +180,16 @@ struct gnufft_cg_s {
 
 namespace {
 
+// A^H k. On odd grids the adjoint's rounding decides what CG returns, and the
+// sums that do not depend on the samples' order are taken (sector_spread.hip).
+int cg_adjoint(gnufft_cg c, const void* k, float2* out, hipStream_t s) {
+  return gnufft::plan_adjoint(c->plan, k, out, c->coils, GNUFFT_STOP_DEAPODIZATION, gnufft::plan_odd_grid(c->plan), s);
+}
+
 // One CG iteration (the body of the captured graph).
 int cg_iteration(gnufft_cg c, hipStream_t s) {
   CG_ABI(gnufft_forward(c->plan, c->p, c->k, c->coils, GNUFFT_STOP_DEAPODIZATION, s));
-  CG_ABI(gnufft_adjoint(c->plan, c->k, c->Ap, c->coils, GNUFFT_STOP_DEAPODIZATION, s));
+  CG_ABI(cg_adjoint(c, c->k, c->Ap, s));
   hipLaunchKernelGGL(cg_pap_kernel, dim3(kCgBlocks), dim3(kCgThreads), 0, s, c->p, c->Ap, c->alpha, c->n, c->pap,
                      c->rr, c->rr_new);
   hipLaunchKernelGGL(cg_step_kernel, dim3(kCgBlocks), dim3(kCgThreads), 0, s, c->x, c->r, c->p, c->Ap, c->rr,
@@ -274,7 +280,7 @@ int gnufft_cg_solve(gnufft_cg c, const void* kdata, void* x_out, uint32_t iterat
   CG_HIP(hipEventRecord(c->ev_in, caller));
   CG_HIP(hipStreamWaitEvent(s, c->ev_in, 0));
   // right-hand side A^H y, then x = 0, r = p = A^H y, rr = |r|^2
-  CG_ABI(gnufft_adjoint(c->plan, kdata, c->y, c->coils, GNUFFT_STOP_DEAPODIZATION, s));
+  CG_ABI(cg_adjoint(c, kdata, c->y, s));
   hipLaunchKernelGGL(cg_init_kernel, dim3(kCgBlocks), dim3(kCgThreads), 0, s, c->x, c->r, c->p,
                      c->y, c->n, c->rr_new);
   CG_HIP(hipGetLastError());

@@ -263,6 +263,15 @@ namespace gnufft {
 // that a captured graph or a batch may reference is freed or replaced.
 uint64_t plan_generation(const gnufft_plan_s* p);
 
+// Some grid length of the plan is odd: its two directions are not adjoint to
+// each other (sector_spread.hip).
+bool plan_odd_grid(const gnufft_plan_s* p);
+
+// gnufft_adjoint; `sector_sums`: gridding by launch_sector_spread. The first such
+// call after a trajectory was set builds tables (and waits for them).
+int plan_adjoint(gnufft_plan_s* p, const void* kdata, void* out, uint32_t n_coils, int stop, bool sector_sums,
+                 void* stream);
+
 // ---------------------------------------------------------------------------
 // Launchers implemented in the .hip translation units (all asynchronous on
 // `stream`; return hipError_t).
@@ -377,6 +386,36 @@ struct SpreadArgs {
   bool fold_shift;         // store at INVERSE-fftshifted positions
 };
 hipError_t launch_spread(const Geom& g, const SpreadArgs& a, hipStream_t s);
+
+// sector_spread.hip: the gridding of CG-SENSE on grids with an odd length.
+constexpr uint32_t kSumsChunk = 1024;  // samples per chunk (two per thread)
+struct SectorSpreadArgs {
+  const float2* data;     // [coil][...] samples, caller's order
+  long long coil_stride;  // elements between coils of `data`
+  const float* dens;      // square roots of the density weights, caller's order (NULL: none)
+  const float4* taps;     // tap table [dim][M]
+  const uint32_t* idx;    // caller's number of sorted sample s
+  const Chunk* chunks;    // the sectors' samples in runs of at most kSumsChunk
+  const uint32_t* first;  // [sectors + 1] first chunk of a sector
+  const uint32_t* cover_off[3];  // sector_cover of the axes in use
+  const uint2* cover[3];
+  float2* sub;   // [chunk][coil][padded point]
+  float2* grid;  // [coil][Ng], every point written
+  uint32_t n_chunks;
+  int n_coils;
+  bool fold_shift;  // store at INVERSE-fftshifted positions
+};
+// per_cu: workgroups per CU that coil blocks are sized for (0: default)
+hipError_t launch_sector_spread(const Geom& g, const SectorSpreadArgs& a, int per_cu, hipStream_t s);
+size_t sector_sub_elems(const Geom& g);  // of one chunk and coil
+// Per grid index q of an axis, the (sector, padded index) pairs that fall on it:
+// entries off[q] .. off[q + 1], by sector.
+void sector_cover(const Geom& g, int axis, std::vector<uint32_t>* off, std::vector<uint2>* entries);
+
+// gridding.hip
+size_t lds_limit();
+// Padded sector of `cb` coils with room for taps past it, kernel table and positions.
+size_t lane_bytes(const Geom& g, int cb);
 // False for geometries whose padded sector does not fit the LDS of a CU (the
 // interp stages padded sectors; gridding.hip).
 bool spread_supported(const Geom& g);

@@ -329,7 +329,7 @@ __global__ void __launch_bounds__(1024) interp_batch_kernel(const BatchOp* __res
 // ---------------------------------------------------------------------------
 // Dynamic LDS a workgroup may use on the current device (160 KB per CU on
 // gfx950; queried, since launches above 64 KB need the device to allow it).
-static size_t lds_limit() {
+size_t lds_limit() {
   static size_t limit = 0;
   if (limit == 0) {
     int dev = 0, v = 0;
@@ -360,7 +360,7 @@ static size_t record_bytes(const Geom& g, int cb) {
   return kp + (((pd + nx) * cb + 1) & ~(size_t)1) * 8 + (size_t)16 * (((1 + 3 * nx) + 3) & ~3) * 4;
 }
 
-static size_t lane_bytes(const Geom& g, int cb) {
+size_t lane_bytes(const Geom& g, int cb) {
   const size_t P = (size_t)g.P, pd = P * P * (g.dim == 3 ? P : 1);
   const size_t slack = g.dim == 3 ? 2 * P * P + 2 * P + 2 : 2 * P + 2;
   const size_t kp = (size_t)((g.K + 3) & ~3) * 4 + (size_t)((3 * (g.P + 4) + 3) & ~3) * 4;
