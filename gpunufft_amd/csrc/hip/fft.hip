@@ -44,18 +44,15 @@ constexpr int kPerThread = kTileElems / kFftThreads;  // tile elements per threa
 // tile of 16 lines (one workgroup per CU), the same work per thread
 constexpr int kBigThreads = 1024;
 constexpr int kBigTileElems = kPerThread * kBigThreads;
-// Light kernels, for transforms that leave the device short of tiles (2-D
-// grids): 8 elements per thread instead of 16 and as many threads as the tile
+// Light kernels, for transforms that leave the device short of tiles (2-D grids
+// mostly): 8 elements per thread instead of 16 and as many threads as the tile
 // needs; 8 lines per tile of a y / z pass, and of an x pass as few image lines as
 // give 512 tiles. What bounds these passes is the chain of stages in a
 // workgroup (the 22 MB of a 480^2 grid with 12 coils would take 5 us), which
-// half the work per thread shortens. Adjoint and forward transform, full tiles
-// and light: 64^2 osf 2, 1 coil 15.9 -> 12.8 us each; 224^2 osf 1.5, 12 coils
-// 30.3 -> 25.5; 256^2 osf 2, 16 coils 36.1 -> 35.1; 240^2 osf 2, 12 coils
-// 33.0 -> 31.3. With many tiles the wider rows of the full tile win: 315 us
-// (full) and 483 us (light) at 192^3, 8 coils. Lengths with kernels of their own
-// (constant strides) keep them down to one tile per CU: x passes of 512 points
-// take 18 and 16 us, light ones 21 and 18.
+// half the work per thread shortens. axis_light and x_light say where they are
+// taken. Adjoint and forward transform, full tiles and by that rule, over 1068
+// transforms (32 to 384 points at osf 1.25, 1.5 and 2 in 2-D with 1 to 32 coils,
+// 32^3 to 128^3 with 1 to 8): 0.88 of the time in the geometric mean.
 constexpr int kLightPerThread = 8;
 // y / z passes of short lines without kernels of their own (32 lines of up to 128
 // points): half the threads, since a prime stage has a butterfly for few of 512
@@ -63,8 +60,9 @@ constexpr int kLightPerThread = 8;
 // 252 x 240 x 66, 6 coils: 135 -> 94 us a pass (0.32 GB, 67 us at 4.8 TB/s).
 constexpr int kShortThreads = 256;
 constexpr int kLightStripe = 8;
-constexpr uint32_t kLightBlocks = 2048, kLightX = 512;  // tiles of a y / z and of an x pass
-constexpr uint32_t kLightFixed = 256;                   // line lengths with kernels of their own
+constexpr uint32_t kLightBlocks = 2048, kLightX = 512;  // full tiles of a y / z and of an x pass
+constexpr uint32_t kLightFixed = 256;                   // x pass of a length with a kernel of its own
+constexpr uint32_t kPrimeWaves = 4096;  // waves that the device holds at a prime stage's 128 registers
 constexpr int kMaxStripe = 32;    // lines per tile of a y / z pass (256 B rows)
 constexpr int kMaxPix = 4;        // image pixels per thread in the x passes
 constexpr int kMaxLen = kMaxPix * kFftThreads;  // longest transform (2048)
@@ -935,12 +933,44 @@ int light_threads(int elems) {
 }
 
 // Small transforms: fewer image lines per tile of an x pass until there are
-// tiles for two workgroups per CU; returns the light kernel's threads, or 0.
-int x_light(int G0, int lines, int Cg, int* Q) {
+// tiles for two workgroups per CU; returns the light kernel's threads, or 0 where
+// the full tile is faster (light over full, summed over the transforms above):
+//  - a prime stage and more waves than the device holds at once: 1.19 .. 1.86
+//    (525^2, 12 coils: 29.2 and 20.7 us); with fewer waves 0.56 .. 0.90;
+//  - 1024 threads without one: forward 1.04 .. 1.12, adjoint 1.05 .. 1.19 above
+//    4096 waves and 0.92 below; with fewer threads 0.60 .. 0.95;
+//  - a kernel of the length's own against 512 threads or more: 0.94 .. 1.16,
+//    against fewer 0.62 .. 0.98.
+int x_light(int G0, int lines, int Cg, bool adjoint, int* Q) {
+  const bool fixed = fixed_length(G0, true);
   if (Cg * G0 > kLightPerThread * 1024) return 0;
-  if ((uint32_t)((lines + *Q - 1) / *Q) >= (fixed_length(G0, true) ? kLightFixed : kLightX)) return 0;
-  *Q = std::max(1, std::min(*Q, lines / 512));
-  return light_threads(Cg * *Q * G0);
+  if ((uint32_t)((lines + *Q - 1) / *Q) >= (fixed ? kLightFixed : kLightX)) return 0;
+  const int q = std::max(1, std::min(*Q, lines / 512));
+  const int nt = light_threads(Cg * q * G0);
+  const bool few = (uint64_t)((lines + q - 1) / q) * (nt / 64) <= kPrimeWaves;
+  if (prime_radix(G0) && !few) return 0;
+  if (fixed && nt > 256) return 0;
+  if (!prime_radix(G0) && nt == 1024 && !(adjoint && few)) return 0;
+  *Q = q;
+  return nt;
+}
+
+// The light kernel's threads for a y / z pass of `tiles` tiles of kLightStripe lines,
+// or 0 where the full tile (`full` of them) is faster (light over full as above):
+//  - a kernel of the length's own: 0.91 .. 1.41;
+//  - a prime stage: 1.10 .. 1.34 with more waves than the device holds at once
+//    (525^2, 12 coils: 36.3 and 25.9 us), 0.77 .. 1.00 with fewer (of 256
+//    threads or more; short lines 0.97 .. 1.13);
+//  - others: 512 threads or more 0.72 .. 1.02; 256 threads 0.79 .. 0.98 up to 2048
+//    waves, then 1.11 .. 1.21; 128 threads (short lines) 0.95 .. 1.11 and, from 2048
+//    tiles on, 0.83.
+int axis_light(int L, uint64_t full, uint64_t tiles) {
+  if (L > kLightPerThread * 1024 / kLightStripe || full >= kLightBlocks || fixed_length(L, false)) return 0;
+  const int nt = light_threads(L * kLightStripe);
+  const uint64_t waves = tiles * (uint64_t)(nt / 64);
+  if (prime_radix(L)) return nt >= 256 && waves <= kPrimeWaves ? nt : 0;
+  if (nt == 128) return tiles >= 2048 ? nt : 0;
+  return nt > 256 || waves <= 2048 ? nt : 0;
 }
 
 // The stage table of axis a inside the device table buffer.
@@ -964,13 +994,13 @@ bool finish_axis(AxisPass* p, int coils, const FftStage* st, bool light) {
   while ((2 << lg) <= kMaxStripe && (2 << lg) * p->LP <= tile) lg++;
   p->stripe = 1 << lg;
   p->x_tiles = (p->nx + p->stripe - 1) / p->stripe;
-  if (light && p->L <= kLightPerThread * 1024 / kLightStripe &&
-      (uint64_t)coils * p->nob * p->x_tiles < (fixed_length(p->L, false) ? kLightFixed : kLightBlocks)) {
+  const uint64_t rows = (uint64_t)coils * p->nob, full = rows * p->x_tiles;
+  if (light) p->light = axis_light(p->L, full, rows * ((p->nx + kLightStripe - 1) / kLightStripe));
+  if (p->light) {
     p->stripe = kLightStripe;
-    p->light = light_threads(p->L * kLightStripe);
     p->x_tiles = (p->nx + p->stripe - 1) / p->stripe;
   }
-  p->short_lines = light && !p->light && p->L * p->stripe <= kPerThread * kShortThreads ? 1 : 0;
+  p->short_lines = light && full >= kLightBlocks && p->L * p->stripe <= kPerThread * kShortThreads ? 1 : 0;
   p->m_stripe = qdiv_const(p->stripe);
   return true;
 }
@@ -1123,7 +1153,7 @@ bool build_adjoint(const Geom& g, float2* grid, float2* tmp, int coils, const fl
   p.shift0 = g.shift_inv[0];
   p.coils = coils;
   x_tiling(G0, p.N0, coils, &p.Cg, &p.Q);
-  if (light) p.light = x_light(G0, p.lines, p.Cg, &p.Q);
+  if (light) p.light = x_light(G0, p.lines, p.Cg, true, &p.Q);
   p.m_g0 = qdiv_const(G0);
   p.m_n0 = qdiv_const(p.N0);
   p.scale = g.fft_scale;
@@ -1160,7 +1190,7 @@ bool build_forward(const Geom& g, const float2* img, bool img_per_coil, const fl
   f.shift0 = g.shift_inv[0];
   f.coils = coils;
   x_tiling(G0, f.N0, coils, &f.Cg, &f.Q);
-  if (light) f.light = x_light(G0, f.lines, f.Cg, &f.Q);
+  if (light) f.light = x_light(G0, f.lines, f.Cg, false, &f.Q);
   f.m_g0 = qdiv_const(G0);
   f.m_n0 = qdiv_const(f.N0);
   f.m_pad = G0 > f.N0 ? qdiv_const(G0 - f.N0) : 0;
