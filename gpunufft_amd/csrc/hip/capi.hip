@@ -250,8 +250,9 @@ struct gnufft_plan_s {
   WorkList work_runs{};
   int lane_per_cu = 0;  // gnufft_plan_set_workgroups_per_cu (0: default)
   bool cover_ok = true;  // sector_cover_ok
-  // tap table and square roots of the density weights, caller's order
+  // tap table, sorted positions and square roots of the density weights, caller's order
   float4* taps_d = nullptr;
+  uint32_t* pos_d = nullptr;  // sorted position of the caller's sample j (behind the tap table)
   float* dens_sqrt_d = nullptr;
   // adjoint: the tile lists of the trajectory and the scratch slots of tiles
   // with several chunks
@@ -357,6 +358,7 @@ void free_traj(gnufft_plan p) {
   p->runs_d = nullptr;
   p->work_runs = WorkList{};
   p->taps_d = nullptr;
+  p->pos_d = nullptr;
   p->dens_sqrt_d = nullptr;
   p->tile_entries_d = nullptr;
   p->tile_chunks_d = nullptr;
@@ -495,7 +497,8 @@ size_t scratch_bytes(gnufft_plan p, uint32_t coils) {
   return std::max(sub, fft) * sizeof(float2);
 }
 
-int ensure_scratch_bytes(gnufft_plan p, size_t bytes) {
+int ensure_scratch(gnufft_plan p, uint32_t coils) {
+  const size_t bytes = scratch_bytes(p, coils);
   if (p->scratch_cap >= bytes) return GNUFFT_OK;
   p->generation++;
   dfree(p->scratch_d);
@@ -506,8 +509,6 @@ int ensure_scratch_bytes(gnufft_plan p, size_t bytes) {
   p->scratch_cap = bytes;
   return GNUFFT_OK;
 }
-
-int ensure_scratch(gnufft_plan p, uint32_t coils) { return ensure_scratch_bytes(p, scratch_bytes(p, coils)); }
 
 // sub: bytes per coil of the sector sums' sub-grids, where they are used
 uint32_t coil_batch(gnufft_plan p, uint32_t n_coils, size_t sub = 0) {
@@ -661,6 +662,14 @@ std::vector<Chunk> partition_chunks(gnufft_plan p, const uint32_t* sdc, uint32_t
   return runs;
 }
 
+// The tap table of the plan's samples and, behind it, their sorted positions.
+hipError_t alloc_taps(gnufft_plan p) {
+  const size_t M = std::max(p->M, 1u), taps = M * p->g.dim * tap_vec(p->g.kw);
+  const hipError_t e = hipMalloc(&p->taps_d, taps * sizeof(float4) + M * sizeof(uint32_t));
+  if (e == hipSuccess) p->pos_d = reinterpret_cast<uint32_t*>(p->taps_d + taps);
+  return e;
+}
+
 // Work lists from the sector offsets: the interp's sector chunks, and the
 // tap table and tile lists of the adjoint.
 int build_chunks(gnufft_plan p, hipStream_t s) {
@@ -689,7 +698,7 @@ int build_chunks(gnufft_plan p, hipStream_t s) {
     STEP(hipMalloc(&cnt_d, (S + 1) * sizeof(uint32_t)));
     STEP(hipMalloc(&hits_d, (size_t)std::max(M, 1u) * sizeof(uint32_t)));
     STEP(hipMalloc(&hit_off_d, ((size_t)M + 1) * sizeof(uint64_t)));
-    STEP(hipMalloc(&p->taps_d, (size_t)std::max(M, 1u) * g.dim * tap_vec(g.kw) * sizeof(float4)));
+    STEP(alloc_taps(p));
     if (p->dens_sorted_d) STEP(hipMalloc(&p->dens_sqrt_d, (size_t)std::max(M, 1u) * sizeof(float)));
     STEP(hipMalloc(&tile_off_d, ((size_t)n_tiles + 1) * sizeof(uint64_t)));
     STEP(hipMalloc(&tot_d, ((size_t)n_tiles + 1) * sizeof(TileTotals)));
@@ -700,7 +709,8 @@ int build_chunks(gnufft_plan p, hipStream_t s) {
     temp_bytes = std::max(temp_bytes, need);
     STEP(hipMalloc(&temp, temp_bytes ? temp_bytes : 4));
     STEP(count_chunks(p->sdc_d, S, p->chunk, cnt_d, off_d, temp, &temp_bytes, s));
-    STEP(launch_taps(g, p->traj_sorted_d, p->dens_sorted_d, p->idx_d, p->lut_d, p->taps_d, p->dens_sqrt_d, hits_d, s));
+    STEP(launch_taps(g, p->traj_sorted_d, p->dens_sorted_d, p->idx_d, p->lut_d, p->taps_d, p->pos_d, p->dens_sqrt_d,
+                     hits_d, s));
     STEP(scan_counts(temp, &temp_bytes, hits_d, hit_off_d, M, s));
     STEP(hipMemcpyAsync(&total, off_d + S, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     STEP(hipMemcpyAsync(&pairs, hit_off_d + M, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
@@ -807,14 +817,14 @@ int build_short(gnufft_plan p, const float* traj, uint32_t M, const float* dens,
     STEP(hipMalloc(&p->centers_d, (size_t)S * D * 4));
     STEP(hipMalloc(&p->chunks_d, n_chunks * sizeof(Chunk)));
     STEP(hipMalloc(&p->runs_d, n_chunks * sizeof(Chunk)));
-    STEP(hipMalloc(&p->taps_d, (size_t)M * D * tap_vec(g.kw) * sizeof(float4)));
+    STEP(alloc_taps(p));
     STEP(hipMalloc(&p->tile_entries_d, entries * sizeof(uint32_t)));
     STEP(hipMalloc(&p->tile_chunks_d, n_tile_chunks * sizeof(TileChunk)));
     STEP(hipMalloc(&p->tile_tasks_d, t.n_tiles * sizeof(TileTask)));
     t.assigned = p->assigned_d, t.idx = p->idx_d, t.sdc = p->sdc_d, t.centers = p->centers_d;
     t.traj_sorted = p->traj_sorted_d, t.dens_sorted = p->dens_sorted_d;
     t.chunks = p->chunks_d, t.runs = p->runs_d;
-    t.taps = p->taps_d, t.dens_sqrt = p->dens_sqrt_d, t.entries = p->tile_entries_d;
+    t.taps = p->taps_d, t.pos = p->pos_d, t.dens_sqrt = p->dens_sqrt_d, t.entries = p->tile_entries_d;
     t.tile_chunks = p->tile_chunks_d, t.tile_tasks = p->tile_tasks_d;
     t.host = p->short_host;
     STEP(launch_short_tables(g, p->tiles, t, p->short_d + in_b + 2 * words_b, &temp_bytes, s));
@@ -1503,15 +1513,13 @@ int gnufft_spread_sorted(gnufft_plan p, const void* data_sorted, void* grid, uin
   if (!p->sdc_d) return fail(GNUFFT_ERR_STATE, "spread_sorted: no trajectory set");
   hipStream_t s = (hipStream_t)stream;
   const uint32_t cc = coil_batch(p, n_coils);
-  // partial tiles and the samples brought to the caller's order
-  const size_t part = (size_t)p->n_slots * tile_points(p->g.dim) * cc;
-  int rc = ensure_scratch_bytes(p, (part + (size_t)p->M * cc) * sizeof(float2));
+  int rc = ensure_scratch(p, cc);
   if (rc) return rc;
   for (uint32_t c0 = 0; c0 < n_coils; c0 += cc) {
     const uint32_t nc = std::min(cc, n_coils - c0);
-    float2* data = p->scratch_d + part;
-    HIP_TRY(launch_unsort((const float2*)data_sorted + (size_t)c0 * p->M, p->M, p->M, (int)nc, p->idx_d, data, s));
-    SpreadArgs a = spread_args(p, data, (float2*)grid + (size_t)c0 * p->g.Ng, nc);
+    SpreadArgs a = spread_args(p, (const float2*)data_sorted + (size_t)c0 * p->M,
+                               (float2*)grid + (size_t)c0 * p->g.Ng, nc);
+    a.pos = p->pos_d;
     a.fold_shift = false;
     TIMED(p, GNUFFT_T_SPREAD, s, plan_spread(p, a, s));
   }

@@ -294,11 +294,12 @@ hipError_t count_chunks(const uint32_t* sdc, uint32_t S, uint32_t chunk, uint32_
 hipError_t launch_fill_chunks(const uint32_t* sdc, const uint32_t* chunk_off, uint32_t S,
                               uint32_t chunk, Chunk* chunks, hipStream_t s);
 
-// Tap table of the sorted samples (s the caller's sample idx[s]), the square
-// roots of their density weights (dens NULL: none), both in the caller's
-// order, and per caller's sample the number of tiles its taps reach (counts).
+// Tap table of the sorted samples (s the caller's sample idx[s]), their sorted
+// positions (pos[idx[s]] = s), the square roots of their density weights (dens
+// NULL: none), all in the caller's order, and per caller's sample the number of
+// tiles its taps reach (counts).
 hipError_t launch_taps(const Geom& g, const float* crds, const float* dens, const uint32_t* idx, const float* lut,
-                       float4* taps, float* dens_sqrt, uint32_t* counts, hipStream_t s);
+                       float4* taps, uint32_t* pos, float* dens_sqrt, uint32_t* counts, hipStream_t s);
 // Exclusive sums of n counts (n + 1 of them).
 hipError_t scan_counts(void* temp, size_t* temp_bytes, const uint32_t* counts, uint64_t* offs, size_t n,
                        hipStream_t s);
@@ -328,6 +329,7 @@ struct ShortTables {
   Chunk *chunks, *runs;  // room for S + M / chunk each
   // tap table and tile lists
   float4* taps;
+  uint32_t* pos;
   float* dens_sqrt;
   uint32_t* entries;       // room for every pair (short_tables_entries)
   TileChunk* tile_chunks;  // room for n_tiles + entries / 128
@@ -379,6 +381,7 @@ struct SpreadArgs {
   long long coil_stride;   // elements between coils of `data`
   const float* dens;       // square roots of the density weights, caller's order (NULL: none)
   const float4* taps;      // tap table [dim][M]
+  const uint32_t* pos;     // data in sector order: sorted position of the caller's sample j (NULL: caller's order)
   TileList tiles;
   float2* scratch;         // partial tiles [slot][coil][tile point]
   float2* grid;            // [coil][Ng], every point written (no prior zeroing)
@@ -420,9 +423,6 @@ size_t lane_bytes(const Geom& g, int cb);
 // interp stages padded sectors; gridding.hip).
 bool spread_supported(const Geom& g);
 bool padded_sector_fits(const Geom& g, int cb);
-// samples in sector order (sample s is the caller's sorted[s]) -> out [coil][n]
-hipError_t launch_unsort(const float2* data, long long coil_stride, uint32_t n, int n_coils,
-                         const uint32_t* sorted, float2* out, hipStream_t s);
 // False when the padded sectors covering one sector are more than 256 (sector
 // widths far below the kernel width).
 bool sector_cover_ok(const Geom& g);

@@ -273,11 +273,12 @@ __global__ void __launch_bounds__(256) taps_kernel(Geom g, const float* __restri
                                                    const float* __restrict__ dens,
                                                    const uint32_t* __restrict__ idx,
                                                    const float* __restrict__ lut, float4* __restrict__ taps,
-                                                   float* __restrict__ dens_sqrt,
+                                                   uint32_t* __restrict__ pos, float* __restrict__ dens_sqrt,
                                                    uint32_t* __restrict__ counts) {
   const uint32_t s = blockIdx.x * 256 + threadIdx.x;
   if (s >= (uint32_t)g.M) return;
   const uint32_t j = idx[s];
+  pos[j] = s;
   if (dens) dens_sqrt[j] = sqrtf(dens[s]);
   uint32_t n = 1;
 #pragma unroll
@@ -291,13 +292,13 @@ __global__ void __launch_bounds__(256) taps_kernel(Geom g, const float* __restri
 }
 
 hipError_t launch_taps(const Geom& g, const float* crds, const float* dens, const uint32_t* idx, const float* lut,
-                       float4* taps, float* dens_sqrt, uint32_t* counts, hipStream_t s) {
+                       float4* taps, uint32_t* pos, float* dens_sqrt, uint32_t* counts, hipStream_t s) {
   if (g.M == 0) return hipSuccess;
   const bool wide = tap_vec(g.kw) == 2;
   auto kernel = g.dim == 3 ? (wide ? taps_kernel<3, 8> : taps_kernel<3, 4>)
                            : (wide ? taps_kernel<2, 8> : taps_kernel<2, 4>);
-  hipLaunchKernelGGL(kernel, dim3((g.M + 255) / 256), dim3(256), 0, s, g, crds, dens, idx, lut, taps, dens_sqrt,
-                     counts);
+  hipLaunchKernelGGL(kernel, dim3((g.M + 255) / 256), dim3(256), 0, s, g, crds, dens, idx, lut, taps, pos,
+                     dens_sqrt, counts);
   return hipGetLastError();
 }
 
@@ -494,6 +495,7 @@ __global__ void __launch_bounds__(kBlock) short_place_kernel(Geom g, TileList l,
   };
   const uint32_t at = place(sector);
   t.idx[at] = j;
+  t.pos[j] = at;
   for (int d = 0; d < DIM; d++) t.traj_sorted[(size_t)d * M + at] = t.traj[(size_t)d * M + j];
   if (t.dens) t.dens_sorted[at] = t.dens[j];
   each_tile<DIM>(l, r, [&](uint32_t tile) { t.entries[place(t.S + tile) - M] = j; });

@@ -158,7 +158,8 @@ __device__ inline uint32_t tile_weights(const Taps<NX>& t, int t0, int T, int G,
 
 // One workgroup: chunk `ci` of the tile lists, coils [group * NC, ...).
 // NX - 1: weights per axis of the tap table.
-template <int DIM, int NC, int NX>
+// SORTED: the data are in sector order.
+template <int DIM, int NC, int NX, bool SORTED = false>
 __device__ __forceinline__ void tile_spread_body(const Geom& g, const SpreadArgs& a, uint32_t ci, int group) {
   using S = TileShape<DIM, NC>;
   constexpr int ER = S::ER, ST = S::ST;
@@ -213,12 +214,13 @@ __device__ __forceinline__ void tile_spread_body(const Geom& g, const SpreadArgs
       sq[q] = 1.0f;
       if (!has_value || at(r, ve + q * (S::NT / S::PP)) >= n) continue;
       if (dens) sq[q] = a.dens[jv[q]];
+      const uint32_t from = SORTED ? a.pos[jv[q]] : jv[q];
       if (coils > 0) {
-        const float2 t = data[jv[q]];
+        const float2 t = data[from];
         v[q].x = t.x, v[q].y = t.y;
       }
       if (coils > 1) {
-        const float2 t = data[(size_t)a.coil_stride + jv[q]];
+        const float2 t = data[(size_t)a.coil_stride + from];
         v[q].z = t.x, v[q].w = t.y;
       }
     }
@@ -361,12 +363,12 @@ __device__ __forceinline__ void tile_spread_body(const Geom& g, const SpreadArgs
 
 // Four workgroups of 8 waves fill a CU up to 64 registers (two more cost 15 us
 // of 683 at 128^3).
-template <int DIM, int NC, int NX>
+template <int DIM, int NC, int NX, bool SORTED>
 __global__ void __launch_bounds__((TileShape<DIM, NC>::NT))
     __attribute__((amdgpu_waves_per_eu(DIM == 3 && NX == 4 ? 8 : 4))) tile_spread_kernel(Geom g, SpreadArgs a) {
   const uint32_t ci = run_item(blockIdx.x);
   if (ci >= a.tiles.n_chunks) return;
-  tile_spread_body<DIM, NC, NX>(g, a, ci, blockIdx.y);
+  tile_spread_body<DIM, NC, NX, SORTED>(g, a, ci, blockIdx.y);
 }
 
 // Sum of a tile's chunks, in chunk order, into the grid. One workgroup per
@@ -397,14 +399,6 @@ __global__ void __launch_bounds__(256) tile_reduce_kernel(Geom g, SpreadArgs a) 
   tile_reduce_body<DIM>(g, a, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
-// Samples in sector order -> the caller's order: out [coil][n].
-__global__ void __launch_bounds__(256) unsort_kernel(const float2* __restrict__ data, long long coil_stride,
-                                                     uint32_t n, const uint32_t* __restrict__ sorted,
-                                                     float2* __restrict__ out) {
-  const uint32_t s = blockIdx.x * 256u + threadIdx.x;
-  if (s < n) out[(size_t)blockIdx.y * n + sorted[s]] = data[(size_t)blockIdx.y * coil_stride + s];
-}
-
 template <typename K>
 hipError_t allow_lds(K kernel, size_t lds) {
   if (lds <= 64 * 1024) return hipSuccess;
@@ -415,10 +409,10 @@ hipError_t allow_lds(K kernel, size_t lds) {
 template <int DIM, int NC, int NX>
 hipError_t tile_launch(const Geom& g, const SpreadArgs& a, hipStream_t s) {
   const size_t lds = TileShape<DIM, NC>::lds;
-  hipError_t e = allow_lds(tile_spread_kernel<DIM, NC, NX>, lds);
+  auto kernel = a.pos ? tile_spread_kernel<DIM, NC, NX, true> : tile_spread_kernel<DIM, NC, NX, false>;
+  hipError_t e = allow_lds(kernel, lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((tile_spread_kernel<DIM, NC, NX>),
-                     dim3(run_blocks(a.tiles.n_chunks), (a.n_coils + NC - 1) / NC),
+  hipLaunchKernelGGL(kernel, dim3(run_blocks(a.tiles.n_chunks), (a.n_coils + NC - 1) / NC),
                      dim3(TileShape<DIM, NC>::NT), lds, s, g, a);
   return hipGetLastError();
 }
@@ -433,14 +427,6 @@ hipError_t tile_launch_nc(const Geom& g, const SpreadArgs& a, hipStream_t s) {
 }
 
 }  // namespace
-
-hipError_t launch_unsort(const float2* data, long long coil_stride, uint32_t n, int n_coils,
-                         const uint32_t* sorted, float2* out, hipStream_t s) {
-  if (n == 0 || n_coils == 0) return hipSuccess;
-  hipLaunchKernelGGL(unsort_kernel, dim3((n + 255) / 256, n_coils), dim3(256), 0, s, data, coil_stride, n,
-                     sorted, out);
-  return hipGetLastError();
-}
 
 hipError_t launch_spread(const Geom& g, const SpreadArgs& a, hipStream_t s) {
   if (a.n_coils == 0) return hipSuccess;
