@@ -417,6 +417,10 @@ void sector_cover(const Geom& g, int axis, std::vector<uint32_t>* off, std::vect
 
 // gridding.hip
 size_t lds_limit();
+// Workgroups per CU that a plan without a target of its own sizes its coil groups
+// for: the environment variable GNUFFT_LANE_PER_CU (1 .. 8, read once), else
+// `built_in`.
+int default_per_cu(int built_in);
 // Padded sector of `cb` coils with room for taps past it, kernel table and positions.
 size_t lane_bytes(const Geom& g, int cb);
 // False for geometries whose padded sector does not fit the LDS of a CU (the

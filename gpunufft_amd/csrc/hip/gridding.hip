@@ -33,6 +33,7 @@
 // 256^2.
 
 #include <algorithm>
+#include <cstdlib>
 #include <type_traits>
 
 #include "gnufft_internal.hpp"
@@ -343,6 +344,15 @@ size_t lds_limit() {
   return limit;
 }
 
+int default_per_cu(int built_in) {
+  static const int set = [] {
+    const char* e = getenv("GNUFFT_LANE_PER_CU");
+    const int v = e ? atoi(e) : 0;
+    return v >= 1 && v <= 8 ? v : 0;
+  }();
+  return set ? set : built_in;
+}
+
 template <typename K>
 static hipError_t allow_lds(K kernel, size_t lds) {
   if (lds <= 64 * 1024) return hipSuccess;
@@ -404,7 +414,7 @@ size_t interp_lds_bytes(const Geom& g, int nc, int taps) { return interp_lds(g, 
 // 0.20 ms.
 int interp_coils(const Geom& g, int n_coils, int per_cu) {
   const int t = interp_taps(g.kw);
-  for (int per = per_cu > 0 ? per_cu : 4; per >= 1; per--) {
+  for (int per = per_cu > 0 ? per_cu : default_per_cu(4); per >= 1; per--) {
     int best = 0, least = 0;
     for (int nc = 8; nc >= 1; nc /= 2) {
       if (interp_lds(g, nc, t) > lds_limit() / per || (nc > 1 && nc / 2 >= n_coils)) continue;

@@ -251,7 +251,7 @@ __global__ void __launch_bounds__(256) sector_fold_kernel(Geom g, SectorSpreadAr
 // order of the L1 sums, so it is part of what a solve returns).
 int sums_coils(const Geom& g, int n_coils, int per_cu) {
   const bool quads = quad_sums(g);
-  for (int per = quads && per_cu > 0 ? per_cu : 3; per >= 1; per--)
+  for (int per = !quads ? 3 : per_cu > 0 ? per_cu : default_per_cu(3); per >= 1; per--)
     for (int cb = 4; cb >= 1; cb /= 2) {
       if (cb > 1 && cb / 2 >= n_coils) continue;
       const size_t bytes = quads ? lane_bytes(g, cb) : (size_t)padded_points(g) * cb * 8;

@@ -129,8 +129,10 @@ int gnufft_plan_get_fft(gnufft_plan plan, int* kind);
  * getOptimalGridDim, cuda_utils.hpp:155). Here the interp's workgroups size
  * their coil group (8, 4, 2 or 1 coils of a padded sector in LDS) for n
  * workgroups per CU, falling back to fewer when the sector does not fit:
- * n = 0 restores the default (4), 1..8 sets it for this plan. Results do not
- * depend on it; gpunufft_amd.autotune times it. */
+ * n = 0 restores the default (4, or the GNUFFT_LANE_PER_CU environment
+ * variable), 1..8 sets it for this plan. Results do not depend on it, but for
+ * the last bits of CG-SENSE on grids with an odd length;
+ * gpunufft_amd.autotune times it. */
 int gnufft_plan_set_workgroups_per_cu(gnufft_plan plan, int n);
 
 /* Sector precompute on the device: assignSectors + sort + sectorDataCount +
