@@ -56,20 +56,57 @@ class Request:
         return self.finish - self.arrival
 
     def device_bytes(self):
-        """Estimate of the device memory the request holds while active."""
-        d = len(self.img_dims)
-        Ng = int(np.prod([int(n * self.osf) for n in self.img_dims]))
-        Ni = int(np.prod(self.img_dims))
-        M = self.traj.shape[1]
-        C = self.coils
-        P = self.sector_width + 2 * (self.kernel_width // 2)
-        # grid + FFT work, gridding scratch and tap tables (bounded by padded
-        # sectors), sens, data, CG vectors, tables
-        sectors = int(np.prod([math.ceil(int(n * self.osf) / self.sector_width)
-                               for n in self.img_dims]))
-        scratch = (sectors + M // 1024 + 1) * C * P ** d * 8
-        return (2 * Ng * C * 8 + scratch + C * Ni * 8 + 2 * C * M * 8 + 5 * Ni * 8 +
-                M * (4 * d + 16) + Ni * 4)
+        """Estimate of the most device memory the request takes: while its
+        tables are built, or active."""
+        d, M, C = len(self.img_dims), self.traj.shape[1], self.coils
+        kw, sw = self.kernel_width, self.sector_width
+        G = [int(n * self.osf) for n in self.img_dims]
+        Ng, Ni = math.prod(G), math.prod(int(n) for n in self.img_dims)
+        pad = (sw + 2 * (kw // 2)) ** d
+        vec = 1 if kw <= 3 else 2  # float4 words of a tap table entry
+        width = (16, 8, 4) if d == 3 else (16, 16)  # tiles of the adjoint gridding
+        sectors = math.prod(-(-g // sw) for g in G)
+        tiles = math.prod(-(-g // (4 * w)) * 4 for g, w in zip(G, width))
+        # (tile, sample) pairs: tiles met by kw taps at any phase, and a quarter for
+        # trajectories that favour the tiles' borders
+        pairs = int(1.25 * M * math.prod(1 + (kw - 1) / w for w in width))
+        # the fused FFT's intermediate (rocFFT's work memory: up to the grid)
+        tmp = Ng // G[-1] * int(self.img_dims[-1]) if max(G) < 1024 and all(map(_smooth, G)) else Ng
+        # partial tiles of the lists that are longer than a chunk, within the plan's bound
+        most = 2048 if d == 3 else 512
+        chunk = 128
+        while chunk < most and chunk * 512 < pairs:
+            chunk *= 2
+        partial = min(2 * pairs / chunk * math.prod(width), max(1 << 20, tmp, M / 1024 * pad))
+        keys = (sectors + tiles) * -(-M // 128)
+        if M <= 1 << 18 and sectors + tiles <= 8192 and keys <= 4 << 20:
+            # short tables: room for every tile a sample could meet; the workspace stays
+            entries = M * math.prod(min(-(-g // w), 4 * vec // w + 3) for g, w in zip(G, width))
+            kept, build = M * 4 * (d + 1) + 2 * 4 * keys, 0
+        else:
+            entries, kept = pairs, 0
+            # copies of the input, both sorts' keys, values and temporaries, counts and offsets
+            build = M * (4 * (d + 1) + 4 * 7) + 5 * 4 * pairs
+        # taps, positions, sorted trajectory, density (sorted, square root), index, sector
+        tables = (M * (16 * vec * d + 4 + 4 * d + 8 + 8) + 4 * entries + kept + 32 * (sectors + M // 256) +
+                  40 * (tiles + entries // 128))
+        inputs = M * 4 * (d + 1) + C * M * 8 + C * Ni * 8 + Ni * 8
+        if any(g % 2 for g in G):  # the sector sums of CG on odd grids
+            kept_sums = (min(sectors, M) + M // 1024) * C * pad * 8
+        else:
+            kept_sums = 0
+        active = (C * Ng * 8 + C * int(max(partial, tmp)) * 8 + kept_sums + C * Ni * 8 + Ni * 4 +  # plan
+                  5 * Ni * 8 + C * M * 8)  # solver
+        # (some forty allocations, rounded up to pages of 2 MiB)
+        return tables + inputs + max(build, active) + (40 << 20)
+
+
+def _smooth(n):
+    """Grid lengths of the fused FFT."""
+    for p in (2, 3, 5, 7, 11, 13, 17, 19):
+        while n % p == 0:
+            n //= p
+    return n == 1
 
 
 def serving_mix(n_requests=40, rate_hz=40.0, seed=7, iterations=10, small=False):
