@@ -218,6 +218,12 @@ struct StageTimer {
   }
 };
 
+// Device memory that the next call uses again.
+struct Arena {
+  char* d = nullptr;
+  size_t cap = 0;
+};
+
 }  // namespace
 
 struct gnufft_plan_s {
@@ -252,7 +258,7 @@ struct gnufft_plan_s {
   bool cover_ok = true;  // sector_cover_ok
   // tap table, sorted positions and square roots of the density weights, caller's order
   float4* taps_d = nullptr;
-  uint32_t* pos_d = nullptr;  // sorted position of the caller's sample j (behind the tap table)
+  uint32_t* pos_d = nullptr;  // sorted position of the caller's sample j
   float* dens_sqrt_d = nullptr;
   // adjoint: the tile lists of the trajectory and the scratch slots of tiles
   // with several chunks
@@ -275,11 +281,10 @@ struct gnufft_plan_s {
   // capacity in bytes
   float2* scratch_d = nullptr;
   size_t scratch_cap = 0;
-  // workspace of short trajectories' tables (at most 40 MB) and pinned words
-  // they report through
-  char* short_d = nullptr;
-  size_t short_cap = 0;
-  uint32_t* short_host = nullptr;
+  // memory behind the trajectory's tables (by samples and sectors; the tile lists)
+  // and of their build
+  Arena tables, lists, work_mem, sort_mem;
+  uint32_t* short_host = nullptr;  // pinned words that short trajectories' tables report through
   // sensitivities
   float2* sens_d = nullptr;
   uint32_t n_sens = 0;
@@ -328,22 +333,63 @@ void dfree(void* p) {
 
 size_t round_up_256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-void free_traj(gnufft_plan p) {
+void release(Arena* a) {
+  dfree(a->d);
+  *a = Arena{};
+}
+
+// Room for `bytes`; the contents are lost. Memory that is more than twice that goes
+// back, above kKeepBytes. A free of large memory takes 0.15 to 0.35 ms, as do one of
+// 128 MB and one of 16 MB among several: a trajectory's tables and temporaries in
+// allocations of their own took 2 to 4.5 ms of a set_trajectory of 0.5 M samples
+// that needs 0.6 ms otherwise.
+constexpr size_t kKeepBytes = 64u << 20;
+hipError_t reserve(Arena* a, size_t bytes) {
+  if (a->cap >= bytes && (a->cap <= kKeepBytes || a->cap / 2 <= bytes)) return hipSuccess;
+  release(a);
+  const hipError_t e = hipMalloc((void**)&a->d, bytes);
+  if (e != hipSuccess)
+    a->d = nullptr;
+  else
+    a->cap = bytes;
+  return e;
+}
+
+// Arrays out of an arena, each at a multiple of 256 bytes (no base: their size only).
+struct Carve {
+  char* base;
+  size_t at = 0;
+  template <typename T>
+  T* take(size_t n) {
+    T* q = base ? reinterpret_cast<T*>(base + at) : nullptr;
+    at += round_up_256(n * sizeof(T));
+    return q;
+  }
+};
+
+// `lay` takes its arrays out of the arena, which is made large enough first.
+template <typename F>
+hipError_t lay_out(Arena* a, F lay) {
+  Carve size{nullptr};
+  lay(size);
+  const hipError_t e = reserve(a, size.at);
+  Carve c{a->d};
+  if (e == hipSuccess) lay(c);
+  return e;
+}
+
+// Temporaries of a table build, after it.
+void give_back(gnufft_plan p) {
+  if (p->work_mem.cap > kKeepBytes) release(&p->work_mem);
+  if (p->sort_mem.cap > kKeepBytes) release(&p->sort_mem);
+}
+
+// Ends the plan's trajectory. Its memory stays for the next one; work under way
+// may still read it, so that it waits for the device (as a free would).
+void clear_traj(gnufft_plan p) {
+  if (p->sdc_d) (void)hipDeviceSynchronize();
   p->generation++;
   p->table_generation++;
-  dfree(p->traj_sorted_d);
-  dfree(p->dens_sorted_d);
-  dfree(p->idx_d);
-  dfree(p->assigned_d);
-  dfree(p->sdc_d);
-  dfree(p->centers_d);
-  dfree(p->chunks_d);
-  dfree(p->runs_d);
-  dfree(p->taps_d);
-  dfree(p->dens_sqrt_d);
-  dfree(p->tile_entries_d);
-  dfree(p->tile_chunks_d);
-  dfree(p->tile_tasks_d);
   dfree(p->sums_chunks_d);
   dfree(p->sums_first_d);
   dfree(p->sub_d);
@@ -372,6 +418,15 @@ void free_traj(gnufft_plan p) {
   p->n_chunks = 0;
   p->work = WorkList{};
   p->g.M = 0;
+}
+
+// Ends the plan's trajectory and gives its memory back.
+void free_traj(gnufft_plan p) {
+  clear_traj(p);
+  release(&p->tables);
+  release(&p->lists);
+  release(&p->work_mem);
+  release(&p->sort_mem);
 }
 
 void free_ffts(gnufft_plan p) {
@@ -639,8 +694,8 @@ double partial_budget(gnufft_plan p) {
 }
 
 // XCD ranges of the plan's `total` sector chunks (sdc: the sectors' offsets)
-// and of their runs; returns the runs, the chunks of each sector merged by up
-// to kInterpRun, unless no sector has several.
+// and (3-D) of their runs; returns the runs, the chunks of each sector merged by
+// up to kInterpRun, unless no sector has several.
 std::vector<Chunk> partition_chunks(gnufft_plan p, const uint32_t* sdc, uint32_t total) {
   std::vector<uint32_t> counts, run_counts;
   std::vector<Chunk> runs;
@@ -650,6 +705,7 @@ std::vector<Chunk> partition_chunks(gnufft_plan p, const uint32_t* sdc, uint32_t
   p->n_chunks = total;
   p->work.chunks = p->chunks_d;
   partition_work(counts.data(), total, &p->work);
+  if (p->g.dim != 3) return {};
   const uint64_t run = (uint64_t)p->chunk * kInterpRun;
   for (uint32_t i = 0; i < p->S; i++)
     for (uint64_t b = sdc[i]; b < sdc[i + 1]; b += run) {
@@ -662,12 +718,23 @@ std::vector<Chunk> partition_chunks(gnufft_plan p, const uint32_t* sdc, uint32_t
   return runs;
 }
 
-// The tap table of the plan's samples and, behind it, their sorted positions.
-hipError_t alloc_taps(gnufft_plan p) {
-  const size_t M = std::max(p->M, 1u), taps = M * p->g.dim * tap_vec(p->g.kw);
-  const hipError_t e = hipMalloc(&p->taps_d, taps * sizeof(float4) + M * sizeof(uint32_t));
-  if (e == hipSuccess) p->pos_d = reinterpret_cast<uint32_t*>(p->taps_d + taps);
-  return e;
+// Memory of the tables of M samples (dens: with density weights).
+hipError_t alloc_tables(gnufft_plan p, uint32_t M, bool dens, bool assigned) {
+  const Geom& g = p->g;
+  const size_t D = (size_t)g.dim, n = std::max(M, 1u), chunks = (size_t)p->S + M / p->chunk;
+  return lay_out(&p->tables, [&](Carve& c) {
+    p->taps_d = c.take<float4>(n * D * tap_vec(g.kw));
+    p->pos_d = c.take<uint32_t>(n);
+    p->traj_sorted_d = c.take<float>(n * D);
+    p->idx_d = c.take<uint32_t>(n);
+    p->assigned_d = assigned ? c.take<uint32_t>(n) : nullptr;
+    p->dens_sorted_d = dens ? c.take<float>(n) : nullptr;
+    p->dens_sqrt_d = dens ? c.take<float>(n) : nullptr;
+    p->centers_d = c.take<uint32_t>(p->S * D);
+    p->chunks_d = c.take<Chunk>(chunks);
+    p->runs_d = g.dim == 3 ? c.take<Chunk>(chunks) : nullptr;
+    p->sdc_d = c.take<uint32_t>((size_t)p->S + 1);
+  });
 }
 
 // Work lists from the sector offsets: the interp's sector chunks, and the
@@ -679,11 +746,10 @@ int build_chunks(gnufft_plan p, hipStream_t s) {
   const uint32_t n_tiles = (uint32_t)p->tiles.nt[0] * p->tiles.nt[1] * p->tiles.nt[2];
   int key_bits = 1;
   while ((1ull << key_bits) < n_tiles) key_bits++;
-  uint32_t *off_d = nullptr, *cnt_d = nullptr, *hits_d = nullptr;
-  uint32_t *keys = nullptr, *keys_s = nullptr, *vals = nullptr;
-  uint64_t *hit_off_d = nullptr, *tile_off_d = nullptr;
+  uint32_t *off = nullptr, *cnt = nullptr, *hits = nullptr, *keys = nullptr, *keys_s = nullptr, *vals = nullptr;
+  uint64_t *hit_off = nullptr, *tile_off = nullptr;
   TileTotals* tot_d = nullptr;
-  void *temp = nullptr, *temp2 = nullptr;
+  void* temp = nullptr;
   size_t temp_bytes = 0, need = 0;
   uint32_t total = 0;
   uint64_t pairs = 0;
@@ -694,61 +760,66 @@ int build_chunks(gnufft_plan p, hipStream_t s) {
     hipError_t e;
 #define STEP(x) \
   if ((e = (x)) != hipSuccess) return e
-    STEP(hipMalloc(&off_d, (S + 1) * sizeof(uint32_t)));
-    STEP(hipMalloc(&cnt_d, (S + 1) * sizeof(uint32_t)));
-    STEP(hipMalloc(&hits_d, (size_t)std::max(M, 1u) * sizeof(uint32_t)));
-    STEP(hipMalloc(&hit_off_d, ((size_t)M + 1) * sizeof(uint64_t)));
-    STEP(alloc_taps(p));
-    if (p->dens_sorted_d) STEP(hipMalloc(&p->dens_sqrt_d, (size_t)std::max(M, 1u) * sizeof(float)));
-    STEP(hipMalloc(&tile_off_d, ((size_t)n_tiles + 1) * sizeof(uint64_t)));
-    STEP(hipMalloc(&tot_d, ((size_t)n_tiles + 1) * sizeof(TileTotals)));
-    STEP(count_chunks(p->sdc_d, S, p->chunk, cnt_d, off_d, nullptr, &temp_bytes, s));
-    STEP(scan_counts(nullptr, &need, hits_d, hit_off_d, M, s));
+    STEP(count_chunks(p->sdc_d, S, p->chunk, cnt, off, nullptr, &temp_bytes, s));
+    STEP(scan_counts(nullptr, &need, hits, hit_off, M, s));
     temp_bytes = std::max(temp_bytes, need);
-    STEP(scan_tile_chunks(nullptr, &need, tile_off_d, n_tiles, 1, tot_d, s));
+    STEP(scan_tile_chunks(nullptr, &need, tile_off, n_tiles, 1, tot_d, s));
     temp_bytes = std::max(temp_bytes, need);
-    STEP(hipMalloc(&temp, temp_bytes ? temp_bytes : 4));
-    STEP(count_chunks(p->sdc_d, S, p->chunk, cnt_d, off_d, temp, &temp_bytes, s));
+    STEP(lay_out(&p->work_mem, [&](Carve& c) {
+      off = c.take<uint32_t>((size_t)S + 1);
+      cnt = c.take<uint32_t>((size_t)S + 1);
+      hits = c.take<uint32_t>(std::max(M, 1u));
+      hit_off = c.take<uint64_t>((size_t)M + 1);
+      tile_off = c.take<uint64_t>((size_t)n_tiles + 1);
+      tot_d = c.take<TileTotals>((size_t)n_tiles + 1);
+      temp = c.take<char>(std::max<size_t>(temp_bytes, 4));
+    }));
+    STEP(count_chunks(p->sdc_d, S, p->chunk, cnt, off, temp, &temp_bytes, s));
     STEP(launch_taps(g, p->traj_sorted_d, p->dens_sorted_d, p->idx_d, p->lut_d, p->taps_d, p->pos_d, p->dens_sqrt_d,
-                     hits_d, s));
-    STEP(scan_counts(temp, &temp_bytes, hits_d, hit_off_d, M, s));
-    STEP(hipMemcpyAsync(&total, off_d + S, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    STEP(hipMemcpyAsync(&pairs, hit_off_d + M, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
-    STEP(hipStreamSynchronize(s));
-    const size_t room = (size_t)(pairs ? pairs : 1);
-    STEP(hipMalloc(&p->chunks_d, (size_t)(total ? total : 1) * sizeof(Chunk)));
-    STEP(launch_fill_chunks(p->sdc_d, off_d, S, p->chunk, p->chunks_d, s));
+                     hits, s));
+    STEP(scan_counts(temp, &temp_bytes, hits, hit_off, M, s));
+    STEP(hipMemcpyAsync(&total, off + S, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    STEP(hipMemcpyAsync(&pairs, hit_off + M, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
     STEP(hipMemcpyAsync(sdc.data(), p->sdc_d, sdc.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    STEP(hipMalloc(&keys, room * sizeof(uint32_t)));
-    STEP(hipMalloc(&keys_s, room * sizeof(uint32_t)));
-    STEP(hipMalloc(&vals, room * sizeof(uint32_t)));
-    STEP(hipMalloc(&p->tile_entries_d, room * sizeof(uint32_t)));
-    STEP(launch_emit_pairs(g, p->tiles, p->taps_d, hit_off_d, keys, vals, s));
-    if (pairs) {
-      STEP(sort_tile_pairs(nullptr, &need, keys, keys_s, vals, p->tile_entries_d, pairs, key_bits, s));
-      STEP(hipMalloc(&temp2, need ? need : 4));
-      STEP(sort_tile_pairs(temp2, &need, keys, keys_s, vals, p->tile_entries_d, pairs, key_bits, s));
-    }
-    STEP(launch_tile_offsets(keys_s, pairs, n_tiles, tile_off_d, s));
+    STEP(hipStreamSynchronize(s));
+    STEP(launch_fill_chunks(p->sdc_d, off, S, p->chunk, p->chunks_d, s));
+    const size_t room = (size_t)(pairs ? pairs : 1);
+    chunk = tile_chunk(g.dim, pairs);
+    need = 0;
+    if (pairs) STEP(sort_tile_pairs(nullptr, &need, keys, keys_s, vals, p->tile_entries_d, pairs, key_bits, s));
+    void* sort_temp = nullptr;
+    STEP(lay_out(&p->sort_mem, [&](Carve& c) {
+      keys = c.take<uint32_t>(room);
+      keys_s = c.take<uint32_t>(room);
+      vals = c.take<uint32_t>(room);
+      sort_temp = c.take<char>(std::max<size_t>(need, 4));
+    }));
+    STEP(lay_out(&p->lists, [&](Carve& c) {
+      p->tile_entries_d = c.take<uint32_t>(room);
+      // (a tile has at most one chunk that is not full)
+      p->tile_chunks_d = c.take<TileChunk>((size_t)n_tiles + pairs / chunk);
+      p->tile_tasks_d = c.take<TileTask>(n_tiles);
+    }));
+    STEP(launch_emit_pairs(g, p->tiles, p->taps_d, hit_off, keys, vals, s));
+    if (pairs) STEP(sort_tile_pairs(sort_temp, &need, keys, keys_s, vals, p->tile_entries_d, pairs, key_bits, s));
+    STEP(launch_tile_offsets(keys_s, pairs, n_tiles, tile_off, s));
     // larger chunks when the partial tiles would not stay within their budget
-    for (chunk = tile_chunk(g.dim, pairs);; chunk *= 2) {
-      STEP(scan_tile_chunks(temp, &temp_bytes, tile_off_d, n_tiles, chunk, tot_d, s));
+    for (;; chunk *= 2) {
+      STEP(scan_tile_chunks(temp, &temp_bytes, tile_off, n_tiles, chunk, tot_d, s));
       STEP(hipMemcpyAsync(&tot, tot_d + n_tiles, sizeof(TileTotals), hipMemcpyDeviceToHost, s));
       STEP(hipStreamSynchronize(s));
       if ((double)tot.slots * tile_points(g.dim) <= partial_budget(p) || chunk >= (1u << 30)) break;
     }
-    STEP(hipMalloc(&p->tile_chunks_d, (size_t)tot.chunks * sizeof(TileChunk)));
-    STEP(hipMalloc(&p->tile_tasks_d, (size_t)(tot.tasks ? tot.tasks : 1) * sizeof(TileTask)));
-    STEP(fill_tile_chunks(tile_off_d, n_tiles, chunk, tot_d, p->tile_chunks_d, p->tile_tasks_d, s));
+    STEP(fill_tile_chunks(tile_off, n_tiles, chunk, tot_d, p->tile_chunks_d, p->tile_tasks_d, s));
 #undef STEP
     return hipStreamSynchronize(s);
   };
   const hipError_t e = run();
-  if (e != hipSuccess) (void)hipStreamSynchronize(s);  // copies into locals
-  for (void* q : {(void*)off_d, (void*)cnt_d, (void*)hits_d, (void*)hit_off_d, (void*)keys, (void*)keys_s,
-                  (void*)vals, (void*)tot_d, (void*)tile_off_d, temp, temp2})
-    dfree(q);
-  if (e != hipSuccess) return fail(GNUFFT_ERR_DEVICE, std::string("chunk list: ") + hipGetErrorString(e));
+  if (e != hipSuccess) {
+    (void)hipStreamSynchronize(s);  // copies into locals
+    return fail(e == hipErrorOutOfMemory ? GNUFFT_ERR_OUT_OF_MEMORY : GNUFFT_ERR_DEVICE,
+                std::string("chunk list: ") + hipGetErrorString(e));
+  }
   p->tiles.entries = p->tile_entries_d;
   p->tiles.chunks = p->tile_chunks_d;
   p->tiles.tasks = p->tile_tasks_d;
@@ -757,8 +828,7 @@ int build_chunks(gnufft_plan p, hipStream_t s) {
   p->n_slots = tot.slots;
   const std::vector<Chunk> runs = partition_chunks(p, sdc.data(), total);
   if (!runs.empty()) {
-    int rc = copy_in((void**)&p->runs_d, runs.data(), runs.size() * sizeof(Chunk), GNUFFT_HOST, s);
-    if (rc) return rc;
+    HIP_TRY(hipMemcpyAsync(p->runs_d, runs.data(), runs.size() * sizeof(Chunk), hipMemcpyHostToDevice, s));
     p->work_runs.chunks = p->runs_d;
     HIP_TRY(hipStreamSynchronize(s));
   }
@@ -785,49 +855,36 @@ int build_short(gnufft_plan p, const float* traj, uint32_t M, const float* dens,
 #define STEP(x) \
   if ((e = (x)) != hipSuccess) return e
     STEP(launch_short_tables(g, p->tiles, t, nullptr, &temp_bytes, s));
-    // the workspace: input, counts, offsets, the scan's temporary
-    const size_t in_b = round_up_256(((size_t)D + 1) * M * 4), words_b = round_up_256(words * 4);
-    const size_t need = in_b + 2 * words_b + temp_bytes;
-    if (p->short_cap < need) {
-      dfree(p->short_d);
-      p->short_d = nullptr;
-      p->short_cap = 0;
-      STEP(hipMalloc((void**)&p->short_d, need));
-      p->short_cap = need;
-    }
+    float* in = nullptr;
+    void* temp = nullptr;
+    STEP(lay_out(&p->work_mem, [&](Carve& c) {
+      in = c.take<float>(((size_t)D + 1) * M);
+      t.counts = c.take<uint32_t>(words);
+      t.offs = c.take<uint32_t>(words);
+      temp = c.take<char>(std::max<size_t>(temp_bytes, 4));
+    }));
+    STEP(alloc_tables(p, M, dens != nullptr, true));
+    STEP(lay_out(&p->lists, [&](Carve& c) {
+      p->tile_entries_d = c.take<uint32_t>(entries);
+      p->tile_chunks_d = c.take<TileChunk>(t.n_tiles + entries / 128);
+      p->tile_tasks_d = c.take<TileTask>(t.n_tiles);
+    }));
     if (!p->short_host)
       STEP(hipHostMalloc((void**)&p->short_host, ((size_t)S + 1 + kShortTotals) * 4, hipHostMallocDefault));
-    float* in = reinterpret_cast<float*>(p->short_d);
     const hipMemcpyKind kind = location == GNUFFT_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
     STEP(hipMemcpyAsync(in, traj, (size_t)D * M * 4, kind, s));
     t.traj = in;
     if (dens) {
       STEP(hipMemcpyAsync(in + (size_t)D * M, dens, (size_t)M * 4, kind, s));
       t.dens = in + (size_t)D * M;
-      STEP(hipMalloc(&p->dens_sorted_d, (size_t)M * 4));
-      STEP(hipMalloc(&p->dens_sqrt_d, (size_t)M * 4));
     }
-    t.counts = reinterpret_cast<uint32_t*>(p->short_d + in_b);
-    t.offs = reinterpret_cast<uint32_t*>(p->short_d + in_b + words_b);
-    const size_t n_chunks = (size_t)S + M / t.chunk, n_tile_chunks = t.n_tiles + entries / 128;
-    STEP(hipMalloc(&p->assigned_d, (size_t)M * 4));
-    STEP(hipMalloc(&p->idx_d, (size_t)M * 4));
-    STEP(hipMalloc(&p->traj_sorted_d, (size_t)M * D * 4));
-    STEP(hipMalloc(&p->sdc_d, ((size_t)S + 1) * 4));
-    STEP(hipMalloc(&p->centers_d, (size_t)S * D * 4));
-    STEP(hipMalloc(&p->chunks_d, n_chunks * sizeof(Chunk)));
-    STEP(hipMalloc(&p->runs_d, n_chunks * sizeof(Chunk)));
-    STEP(alloc_taps(p));
-    STEP(hipMalloc(&p->tile_entries_d, entries * sizeof(uint32_t)));
-    STEP(hipMalloc(&p->tile_chunks_d, n_tile_chunks * sizeof(TileChunk)));
-    STEP(hipMalloc(&p->tile_tasks_d, t.n_tiles * sizeof(TileTask)));
     t.assigned = p->assigned_d, t.idx = p->idx_d, t.sdc = p->sdc_d, t.centers = p->centers_d;
     t.traj_sorted = p->traj_sorted_d, t.dens_sorted = p->dens_sorted_d;
     t.chunks = p->chunks_d, t.runs = p->runs_d;
     t.taps = p->taps_d, t.pos = p->pos_d, t.dens_sqrt = p->dens_sqrt_d, t.entries = p->tile_entries_d;
     t.tile_chunks = p->tile_chunks_d, t.tile_tasks = p->tile_tasks_d;
     t.host = p->short_host;
-    STEP(launch_short_tables(g, p->tiles, t, p->short_d + in_b + 2 * words_b, &temp_bytes, s));
+    STEP(launch_short_tables(g, p->tiles, t, temp, &temp_bytes, s));
 #undef STEP
     return hipSuccess;
   };
@@ -1187,7 +1244,6 @@ int gnufft_plan_destroy(gnufft_plan p) {
   free_traj(p);
   free_ffts(p);
   dfree(p->scratch_d);
-  dfree(p->short_d);
   if (p->short_host) (void)hipHostFree(p->short_host);
   for (int a = 0; a < 3; a++) {
     dfree(p->cover_off_d[a]);
@@ -1235,64 +1291,61 @@ int gnufft_plan_set_trajectory(gnufft_plan p, const float* traj, uint32_t n_samp
                                const float* dens, int location, void* stream) {
   if (!p || (!traj && n_samples)) return fail(GNUFFT_ERR_INVALID_ARGUMENT, "set_trajectory: null");
   hipStream_t s = (hipStream_t)stream;
-  free_traj(p);
+  clear_traj(p);
   const uint32_t M = n_samples;
   const int D = p->g.dim;
   if (short_tables_ok(M, p->S, (uint32_t)p->tiles.nt[0] * p->tiles.nt[1] * p->tiles.nt[2])) {
     const int rc = build_short(p, traj, M, dens, location, s);
     if (rc != GNUFFT_OK) free_traj(p);
+    give_back(p);
     return rc;
   }
-  float* traj_in = nullptr;
-  float* dens_in = nullptr;
-  uint32_t *keys = nullptr, *vals = nullptr, *keys_sorted = nullptr;
+  float *traj_in = nullptr, *dens_in = nullptr;
+  uint32_t *vals = nullptr, *keys_sorted = nullptr;
   void* temp = nullptr;
-  int rc = GNUFFT_OK;
-  hipError_t e = hipSuccess;
   size_t temp_bytes = 0;
   int key_bits = 1;
   while ((1ull << key_bits) < (unsigned long long)p->S) key_bits++;
-
-  rc = copy_in((void**)&traj_in, traj, (size_t)D * M * sizeof(float), location, s);
-  if (rc == GNUFFT_OK && dens) rc = copy_in((void**)&dens_in, dens, (size_t)M * 4, location, s);
-  if (rc != GNUFFT_OK) goto done;
-  e = hipMalloc(&keys, (size_t)(M ? M : 1) * 4);
-  if (e == hipSuccess) e = hipMalloc(&vals, (size_t)(M ? M : 1) * 4);
-  if (e == hipSuccess) e = hipMalloc(&keys_sorted, (size_t)(M ? M : 1) * 4);
-  if (e == hipSuccess) e = hipMalloc(&p->idx_d, (size_t)(M ? M : 1) * 4);
-  if (e == hipSuccess) e = hipMalloc(&p->traj_sorted_d, (size_t)(M ? M : 1) * D * 4);
-  if (e == hipSuccess && dens) e = hipMalloc(&p->dens_sorted_d, (size_t)(M ? M : 1) * 4);
-  if (e == hipSuccess) e = hipMalloc(&p->sdc_d, (size_t)(p->S + 1) * 4);
-  if (e == hipSuccess) e = hipMalloc(&p->centers_d, (size_t)p->S * D * 4);
+  auto run = [&]() -> hipError_t {
+    hipError_t e;
+#define STEP(x) \
+  if ((e = (x)) != hipSuccess) return e
+    STEP(alloc_tables(p, M, dens != nullptr, true));
+    if (M) STEP(sort_pairs(nullptr, &temp_bytes, p->assigned_d, keys_sorted, vals, p->idx_d, M, key_bits, s));
+    // (the sort's temporaries: build_chunks uses the memory again)
+    const size_t n = std::max(M, 1u);
+    STEP(lay_out(&p->work_mem, [&](Carve& c) {
+      traj_in = c.take<float>(n * D);
+      dens_in = dens ? c.take<float>(n) : nullptr;
+      vals = c.take<uint32_t>(n);
+      keys_sorted = c.take<uint32_t>(n);
+      temp = c.take<char>(std::max<size_t>(temp_bytes, 4));
+    }));
+    const hipMemcpyKind kind = location == GNUFFT_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
+    if (M) STEP(hipMemcpyAsync(traj_in, traj, (size_t)D * M * 4, kind, s));
+    if (M && dens) STEP(hipMemcpyAsync(dens_in, dens, (size_t)M * 4, kind, s));
+    STEP(launch_assign_sectors(p->g, traj_in, M, p->assigned_d, vals, s));
+    if (M) STEP(sort_pairs(temp, &temp_bytes, p->assigned_d, keys_sorted, vals, p->idx_d, M, key_bits, s));
+    STEP(launch_sector_data_count(keys_sorted, M, p->S, p->sdc_d, s));
+    STEP(launch_sector_centers(p->g, p->centers_d, s));
+    STEP(launch_gather_traj(traj_in, dens_in, p->idx_d, M, D, p->traj_sorted_d, p->dens_sorted_d, s));
+#undef STEP
+    return hipSuccess;
+  };
+  hipError_t e = run();
+  const hipError_t waited = hipStreamSynchronize(s);
+  if (e == hipSuccess) e = waited;
+  int rc = GNUFFT_OK;
   if (e != hipSuccess) {
-    rc = fail(GNUFFT_ERR_OUT_OF_MEMORY, std::string("set_trajectory: ") + hipGetErrorString(e));
-    goto done;
+    rc = fail(e == hipErrorOutOfMemory ? GNUFFT_ERR_OUT_OF_MEMORY : GNUFFT_ERR_DEVICE,
+              std::string("set_trajectory: ") + hipGetErrorString(e));
+  } else {
+    p->M = M;
+    p->g.M = (int)M;
+    rc = build_chunks(p, s);
   }
-  e = launch_assign_sectors(p->g, traj_in, M, keys, vals, s);
-  if (e == hipSuccess && M) e = sort_pairs(nullptr, &temp_bytes, keys, keys_sorted, vals, p->idx_d, M, key_bits, s);
-  if (e == hipSuccess) e = hipMalloc(&temp, temp_bytes ? temp_bytes : 4);
-  if (e == hipSuccess && M) e = sort_pairs(temp, &temp_bytes, keys, keys_sorted, vals, p->idx_d, M, key_bits, s);
-  if (e == hipSuccess) e = launch_sector_data_count(keys_sorted, M, p->S, p->sdc_d, s);
-  if (e == hipSuccess) e = launch_sector_centers(p->g, p->centers_d, s);
-  if (e == hipSuccess) e = launch_gather_traj(traj_in, dens_in, p->idx_d, M, D, p->traj_sorted_d, p->dens_sorted_d, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  if (e != hipSuccess) {
-    rc = fail(GNUFFT_ERR_DEVICE, std::string("set_trajectory: ") + hipGetErrorString(e));
-    goto done;
-  }
-  p->assigned_d = keys;
-  keys = nullptr;
-  p->M = M;
-  p->g.M = (int)M;
-  rc = build_chunks(p, s);
-done:
-  dfree(traj_in);
-  dfree(dens_in);
-  dfree(keys);
-  dfree(vals);
-  dfree(keys_sorted);
-  dfree(temp);
   if (rc != GNUFFT_OK) free_traj(p);
+  give_back(p);
   return rc;
 }
 
@@ -1400,24 +1453,31 @@ int gnufft_plan_load_precomputed(gnufft_plan p, const float* traj_sorted,
     int rc = gnufft_check_precomputed(dims, p->sw, p->osf, tr_h, di_h, sdc_h, cen_h, M);
     if (rc) return rc;
   }
-  free_traj(p);
-  int rc = copy_in((void**)&p->traj_sorted_d, traj_sorted, (size_t)D * M * 4, location, s);
-  if (!rc) rc = copy_in((void**)&p->idx_d, data_indices, (size_t)M * 4, location, s);
-  if (!rc) rc = copy_in((void**)&p->sdc_d, sector_data_count, (size_t)(p->S + 1) * 4, location, s);
-  if (!rc) rc = copy_in((void**)&p->centers_d, sector_centers, (size_t)p->S * D * 4, location, s);
-  if (!rc && dens_sorted) rc = copy_in((void**)&p->dens_sorted_d, dens_sorted, (size_t)M * 4, location, s);
-  if (!rc && deapo)
-    HIP_TRY(hipMemcpyAsync(p->deapo_d, deapo, (size_t)p->g.Ni * 4,
-                           location == GNUFFT_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice,
-                           s));
-  if (!rc && hipStreamSynchronize(s) != hipSuccess)
-    rc = fail(GNUFFT_ERR_DEVICE, "load_precomputed: table upload");
-  if (!rc) {
+  clear_traj(p);
+  const hipMemcpyKind kind = location == GNUFFT_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
+  hipError_t e = alloc_tables(p, M, dens_sorted != nullptr, false);
+  auto copy = [&](void* dst, const void* src, size_t bytes) {
+    if (e == hipSuccess && bytes) e = hipMemcpyAsync(dst, src, bytes, kind, s);
+  };
+  copy(p->traj_sorted_d, traj_sorted, (size_t)D * M * 4);
+  copy(p->idx_d, data_indices, (size_t)M * 4);
+  copy(p->sdc_d, sector_data_count, (size_t)(p->S + 1) * 4);
+  copy(p->centers_d, sector_centers, (size_t)p->S * D * 4);
+  if (dens_sorted) copy(p->dens_sorted_d, dens_sorted, (size_t)M * 4);
+  if (deapo) copy(p->deapo_d, deapo, (size_t)p->g.Ni * 4);
+  const hipError_t waited = hipStreamSynchronize(s);
+  if (e == hipSuccess) e = waited;
+  int rc = GNUFFT_OK;
+  if (e != hipSuccess) {
+    rc = fail(e == hipErrorOutOfMemory ? GNUFFT_ERR_OUT_OF_MEMORY : GNUFFT_ERR_DEVICE,
+              std::string("load_precomputed: ") + hipGetErrorString(e));
+  } else {
     p->M = M;
     p->g.M = (int)M;
     rc = build_chunks(p, s);
   }
   if (rc) free_traj(p);
+  give_back(p);
   return rc;
 }
 

@@ -548,8 +548,8 @@ __global__ void __launch_bounds__(1024) short_lists_kernel(Geom g, ShortTables t
   for (uint32_t s = s0; s < s1; s++) {
     const uint32_t b = off(s), e = off(s + 1);
     for (uint32_t p = b; p < e; p += t.chunk) t.chunks[at.x++] = Chunk{s, p, min(p + t.chunk, e), 0};
-    for (uint32_t p = b; p < e; p += t.chunk * kInterpRun)
-      t.runs[at.y++] = Chunk{s, p, min(p + t.chunk * kInterpRun, e), 0};
+    if (DIM == 3)
+      for (uint32_t p = b; p < e; p += t.chunk * kInterpRun) t.runs[at.y++] = Chunk{s, p, min(p + t.chunk * kInterpRun, e), 0};
   }
   uint32_t* totals = t.host + S + 1;
   if (tid == 0) totals[0] = all.x, totals[1] = all.y;

@@ -80,25 +80,27 @@ class Request:
         partial = min(2 * pairs / chunk * math.prod(width), max(1 << 20, tmp, M / 1024 * pad))
         keys = (sectors + tiles) * -(-M // 128)
         if M <= 1 << 18 and sectors + tiles <= 8192 and keys <= 4 << 20:
-            # short tables: room for every tile a sample could meet; the workspace stays
+            # short tables: room for every tile a sample could meet
             entries = M * math.prod(min(-(-g // w), 4 * vec // w + 3) for g, w in zip(G, width))
-            kept, build = M * 4 * (d + 1) + 2 * 4 * keys, 0
+            build = [M * 4 * (d + 1) + 2 * 4 * keys]
         else:
-            entries, kept = pairs, 0
-            # copies of the input, both sorts' keys, values and temporaries, counts and offsets
-            build = M * (4 * (d + 1) + 4 * 7) + 5 * 4 * pairs
+            entries = pairs
+            # copies of the input and the first sort, then counts and offsets; the
+            # pairs' keys, values and sort
+            build = [max(M * (4 * (d + 1) + 4 * 4), M * 12), 5 * 4 * pairs]
+        kept = sum(b for b in build if b <= 64 << 20)  # (larger temporaries are given back)
         # taps, positions, sorted trajectory, density (sorted, square root), index, sector
-        tables = (M * (16 * vec * d + 4 + 4 * d + 8 + 8) + 4 * entries + kept + 32 * (sectors + M // 256) +
+        tables = (M * (16 * vec * d + 4 + 4 * d + 8 + 8) + 4 * entries + 32 * (sectors + M // 256) +
                   40 * (tiles + entries // 128))
         inputs = M * 4 * (d + 1) + C * M * 8 + C * Ni * 8 + Ni * 8
         if any(g % 2 for g in G):  # the sector sums of CG on odd grids
-            kept_sums = (min(sectors, M) + M // 1024) * C * pad * 8
+            sums = (min(sectors, M) + M // 1024) * C * pad * 8
         else:
-            kept_sums = 0
-        active = (C * Ng * 8 + C * int(max(partial, tmp)) * 8 + kept_sums + C * Ni * 8 + Ni * 4 +  # plan
+            sums = 0
+        active = (C * Ng * 8 + C * int(max(partial, tmp)) * 8 + sums + C * Ni * 8 + Ni * 4 +  # plan
                   5 * Ni * 8 + C * M * 8)  # solver
         # (some forty allocations, rounded up to pages of 2 MiB)
-        return tables + inputs + max(build, active) + (40 << 20)
+        return tables + inputs + max(sum(build), active + kept) + (40 << 20)
 
 
 def _smooth(n):
