@@ -38,13 +38,19 @@ hipError_t launch_assign_sectors(const Geom& g, const float* traj, uint32_t M, u
   return hipGetLastError();
 }
 
+// Radix passes at every size: below a million pairs the library's default is a merge
+// sort of some 24 launches, twice a trajectory on the long path, where 16 bits of
+// keys need two radix passes.
+using SortConfig = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config,
+                                              rocprim::default_config, 0>;
+
 // Stable LSD radix sort of (sector, original index) pairs: within a sector
 // samples keep their original order, the canonical order of the reference's
 // std::sort (equal per-sector index sets, CUDA/src/gpuNUFFT_operator_factory.cpp:56-72).
 hipError_t sort_pairs(void* temp, size_t* temp_bytes, const uint32_t* keys_in,
                       uint32_t* keys_out, const uint32_t* vals_in, uint32_t* vals_out,
                       uint32_t M, int key_bits, hipStream_t s) {
-  return rocprim::radix_sort_pairs(temp, *temp_bytes, keys_in, keys_out, vals_in, vals_out,
+  return rocprim::radix_sort_pairs<SortConfig>(temp, *temp_bytes, keys_in, keys_out, vals_in, vals_out,
                                    (size_t)M, 0, key_bits, s);
 }
 
@@ -344,7 +350,7 @@ hipError_t launch_emit_pairs(const Geom& g, const TileList& l, const float4* tap
 
 hipError_t sort_tile_pairs(void* temp, size_t* temp_bytes, const uint32_t* keys_in, uint32_t* keys_out,
                            const uint32_t* vals_in, uint32_t* vals_out, size_t n, int key_bits, hipStream_t s) {
-  return rocprim::radix_sort_pairs(temp, *temp_bytes, keys_in, keys_out, vals_in, vals_out, n, 0, key_bits, s);
+  return rocprim::radix_sort_pairs<SortConfig>(temp, *temp_bytes, keys_in, keys_out, vals_in, vals_out, n, 0, key_bits, s);
 }
 
 // Offset of tile t: lower bound of its key.
