@@ -79,7 +79,7 @@ class Request:
             chunk *= 2
         partial = min(2 * pairs / chunk * math.prod(width), max(1 << 20, tmp, M / 1024 * pad))
         keys = (sectors + tiles) * -(-M // 128)
-        if M <= 1 << 18 and sectors + tiles <= 8192 and keys <= 4 << 20:
+        if M <= 1 << 18 and sectors + tiles <= 8192 and keys <= 6 << 20:
             # short tables: room for every tile a sample could meet
             entries = M * math.prod(min(-(-g // w), 4 * vec // w + 3) for g, w in zip(G, width))
             build = [M * 4 * (d + 1) + 2 * 4 * keys]
