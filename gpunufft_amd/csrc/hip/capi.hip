@@ -284,7 +284,7 @@ struct gnufft_plan_s {
   // memory behind the trajectory's tables (by samples and sectors; the tile lists)
   // and of their build
   Arena tables, lists, work_mem, sort_mem;
-  uint32_t* short_host = nullptr;  // pinned words that short trajectories' tables report through
+  uint32_t* host_words = nullptr;  // pinned words that the build reports through (ensure_host)
   // sensitivities
   float2* sens_d = nullptr;
   uint32_t n_sens = 0;
@@ -342,7 +342,7 @@ void release(Arena* a) {
 // back, above kKeepBytes. A free of large memory takes 0.15 to 0.35 ms, as do one of
 // 128 MB and one of 16 MB among several: a trajectory's tables and temporaries in
 // allocations of their own took 2 to 4.5 ms of a set_trajectory of 0.5 M samples
-// that needs 0.6 ms otherwise.
+// that needs 0.4 ms otherwise.
 constexpr size_t kKeepBytes = 64u << 20;
 hipError_t reserve(Arena* a, size_t bytes) {
   if (a->cap >= bytes && (a->cap <= kKeepBytes || a->cap / 2 <= bytes)) return hipSuccess;
@@ -718,6 +718,14 @@ std::vector<Chunk> partition_chunks(gnufft_plan p, const uint32_t* sdc, uint32_t
   return runs;
 }
 
+// Room for the sectors' offsets and some totals in pinned memory (a copy of a few
+// words to pageable memory takes 20 us, of 4097 words 60).
+hipError_t ensure_host(gnufft_plan p) {
+  static_assert(kShortTotals <= 8, "totals of either build");
+  if (p->host_words) return hipSuccess;
+  return hipHostMalloc((void**)&p->host_words, ((size_t)p->S + 1 + 1 + 8) * 4, hipHostMallocDefault);
+}
+
 // Memory of the tables of M samples (dens: with density weights).
 hipError_t alloc_tables(gnufft_plan p, uint32_t M, bool dens, bool assigned) {
   const Geom& g = p->g;
@@ -751,11 +759,9 @@ int build_chunks(gnufft_plan p, hipStream_t s) {
   TileTotals* tot_d = nullptr;
   void* temp = nullptr;
   size_t temp_bytes = 0, need = 0;
-  uint32_t total = 0;
+  uint32_t total = 0, chunk = 0;
   uint64_t pairs = 0;
   TileTotals tot{0, 0, 0};
-  uint32_t chunk = 0;
-  std::vector<uint32_t> sdc((size_t)S + 1);
   auto run = [&]() -> hipError_t {
     hipError_t e;
 #define STEP(x) \
@@ -778,10 +784,14 @@ int build_chunks(gnufft_plan p, hipStream_t s) {
     STEP(launch_taps(g, p->traj_sorted_d, p->dens_sorted_d, p->idx_d, p->lut_d, p->taps_d, p->pos_d, p->dens_sqrt_d,
                      hits, s));
     STEP(scan_counts(temp, &temp_bytes, hits, hit_off, M, s));
-    STEP(hipMemcpyAsync(&total, off + S, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    STEP(hipMemcpyAsync(&pairs, hit_off + M, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
-    STEP(hipMemcpyAsync(sdc.data(), p->sdc_d, sdc.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    STEP(ensure_host(p));
+    uint32_t* words = p->host_words + S + 1 + (S + 1) % 2;  // pairs, chunks, tile totals
+    STEP(hipMemcpyAsync(words, hit_off + M, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+    STEP(hipMemcpyAsync(words + 2, off + S, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    STEP(hipMemcpyAsync(p->host_words, p->sdc_d, ((size_t)S + 1) * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     STEP(hipStreamSynchronize(s));
+    memcpy(&pairs, words, sizeof(pairs));
+    total = words[2];
     STEP(launch_fill_chunks(p->sdc_d, off, S, p->chunk, p->chunks_d, s));
     const size_t room = (size_t)(pairs ? pairs : 1);
     chunk = tile_chunk(g.dim, pairs);
@@ -806,8 +816,9 @@ int build_chunks(gnufft_plan p, hipStream_t s) {
     // larger chunks when the partial tiles would not stay within their budget
     for (;; chunk *= 2) {
       STEP(scan_tile_chunks(temp, &temp_bytes, tile_off, n_tiles, chunk, tot_d, s));
-      STEP(hipMemcpyAsync(&tot, tot_d + n_tiles, sizeof(TileTotals), hipMemcpyDeviceToHost, s));
+      STEP(hipMemcpyAsync(words + 3, tot_d + n_tiles, sizeof(TileTotals), hipMemcpyDeviceToHost, s));
       STEP(hipStreamSynchronize(s));
+      memcpy(&tot, words + 3, sizeof(tot));
       if ((double)tot.slots * tile_points(g.dim) <= partial_budget(p) || chunk >= (1u << 30)) break;
     }
     STEP(fill_tile_chunks(tile_off, n_tiles, chunk, tot_d, p->tile_chunks_d, p->tile_tasks_d, s));
@@ -816,7 +827,7 @@ int build_chunks(gnufft_plan p, hipStream_t s) {
   };
   const hipError_t e = run();
   if (e != hipSuccess) {
-    (void)hipStreamSynchronize(s);  // copies into locals
+    (void)hipStreamSynchronize(s);  // copies into the pinned words
     return fail(e == hipErrorOutOfMemory ? GNUFFT_ERR_OUT_OF_MEMORY : GNUFFT_ERR_DEVICE,
                 std::string("chunk list: ") + hipGetErrorString(e));
   }
@@ -826,7 +837,7 @@ int build_chunks(gnufft_plan p, hipStream_t s) {
   p->tiles.n_chunks = tot.chunks;
   p->tiles.n_tasks = tot.tasks;
   p->n_slots = tot.slots;
-  const std::vector<Chunk> runs = partition_chunks(p, sdc.data(), total);
+  const std::vector<Chunk> runs = partition_chunks(p, p->host_words, total);
   if (!runs.empty()) {
     HIP_TRY(hipMemcpyAsync(p->runs_d, runs.data(), runs.size() * sizeof(Chunk), hipMemcpyHostToDevice, s));
     p->work_runs.chunks = p->runs_d;
@@ -869,8 +880,7 @@ int build_short(gnufft_plan p, const float* traj, uint32_t M, const float* dens,
       p->tile_chunks_d = c.take<TileChunk>(t.n_tiles + entries / 128);
       p->tile_tasks_d = c.take<TileTask>(t.n_tiles);
     }));
-    if (!p->short_host)
-      STEP(hipHostMalloc((void**)&p->short_host, ((size_t)S + 1 + kShortTotals) * 4, hipHostMallocDefault));
+    STEP(ensure_host(p));
     const hipMemcpyKind kind = location == GNUFFT_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
     STEP(hipMemcpyAsync(in, traj, (size_t)D * M * 4, kind, s));
     t.traj = in;
@@ -883,7 +893,7 @@ int build_short(gnufft_plan p, const float* traj, uint32_t M, const float* dens,
     t.chunks = p->chunks_d, t.runs = p->runs_d;
     t.taps = p->taps_d, t.pos = p->pos_d, t.dens_sqrt = p->dens_sqrt_d, t.entries = p->tile_entries_d;
     t.tile_chunks = p->tile_chunks_d, t.tile_tasks = p->tile_tasks_d;
-    t.host = p->short_host;
+    t.host = p->host_words;
     STEP(launch_short_tables(g, p->tiles, t, temp, &temp_bytes, s));
 #undef STEP
     return hipSuccess;
@@ -894,14 +904,14 @@ int build_short(gnufft_plan p, const float* traj, uint32_t M, const float* dens,
   if (e != hipSuccess)
     return fail(e == hipErrorOutOfMemory ? GNUFFT_ERR_OUT_OF_MEMORY : GNUFFT_ERR_DEVICE,
                 std::string("set_trajectory: ") + hipGetErrorString(e));
-  const uint32_t* totals = p->short_host + S + 1;
+  const uint32_t* totals = p->host_words + S + 1;
   p->tiles.entries = p->tile_entries_d;
   p->tiles.chunks = p->tile_chunks_d;
   p->tiles.tasks = p->tile_tasks_d;
   p->tiles.n_chunks = totals[2];
   p->n_slots = totals[3];
   p->tiles.n_tasks = totals[4];
-  if (!partition_chunks(p, p->short_host, totals[0]).empty()) p->work_runs.chunks = p->runs_d;
+  if (!partition_chunks(p, p->host_words, totals[0]).empty()) p->work_runs.chunks = p->runs_d;
   return GNUFFT_OK;
 }
 
@@ -1244,7 +1254,7 @@ int gnufft_plan_destroy(gnufft_plan p) {
   free_traj(p);
   free_ffts(p);
   dfree(p->scratch_d);
-  if (p->short_host) (void)hipHostFree(p->short_host);
+  if (p->host_words) (void)hipHostFree(p->host_words);
   for (int a = 0; a < 3; a++) {
     dfree(p->cover_off_d[a]);
     dfree(p->cover_d[a]);
