@@ -828,9 +828,48 @@ __global__ void __launch_bounds__(kFftThreads, 4) fft_forward_first_batch_kernel
 // ---------------------------------------------------------------------------
 uint32_t qdiv_const(int d) { return d == 1 ? 0u : udiv_magic((uint32_t)d); }
 
+// Line lengths with compile-time kernels: (L, tile lines of a y / z pass,
+// radices). The tile must be the one finish_axis picks for L. Besides the
+// common smooth lengths (and 320, the 160^3 osf-2 grid), the 3-D grids of
+// 96^3 .. 160^3 images at osf 1.5 and 2: those with a prime factor 7 .. 19
+// and the smooth ones that need four stages (144, 180, 216, 240, 288).
+#define GNUFFT_FIXED_FFT_SIZES(X) \
+  X(96, 32, 8, 4, 3)              \
+  X(128, 32, 8, 8, 2)             \
+  X(160, 32, 8, 4, 5)             \
+  X(192, 32, 8, 8, 3)             \
+  X(256, 16, 8, 8, 4)             \
+  X(156, 32, 4, 3, 13)            \
+  X(168, 32, 8, 3, 7)             \
+  X(204, 32, 4, 3, 17)            \
+  X(208, 32, 8, 2, 13)            \
+  X(224, 32, 8, 4, 7)             \
+  X(228, 32, 4, 3, 19)            \
+  X(272, 16, 8, 2, 17)            \
+  X(304, 16, 8, 2, 19)            \
+  X(320, 16, 8, 8, 5)             \
+  X(144, 32, 4, 4, 3, 3)          \
+  X(180, 32, 4, 5, 3, 3)          \
+  X(216, 32, 8, 3, 3, 3)          \
+  X(240, 32, 4, 4, 5, 3)          \
+  X(288, 16, 8, 4, 3, 3)
+
+// Line lengths with compile-time kernels for the x passes only (their y / z
+// passes use the large tiles).
+#define GNUFFT_FIXED_X_SIZES(X) \
+  X(512, 0, 8, 8, 8)
+
+// Stages of a line. Lengths with kernels of their own take those kernels' stages, so
+// that every kernel gives the same bits.
 bool make_radices(int L, FftRadices* rad) {
   rad->n = 0;
   int n = L;
+#define GNUFFT_LENGTH_CASE(LEN, TILE, ...) \
+  if (L == LEN)                            \
+    for (int r : {__VA_ARGS__}) rad->st[rad->n++].R = r, n /= r;
+  GNUFFT_FIXED_FFT_SIZES(GNUFFT_LENGTH_CASE)
+  GNUFFT_FIXED_X_SIZES(GNUFFT_LENGTH_CASE)
+#undef GNUFFT_LENGTH_CASE
   const int order[10] = {8, 4, 2, 3, 5, 7, 11, 13, 17, 19};
   for (int r : order)
     while (n > 1 && n % r == 0) {
@@ -882,37 +921,6 @@ void x_tiling(int G0, int N0, int coils, int* Cg, int* Q) {
   *Q = std::max(1, std::min(per_tile / *Cg, (kMaxPix * kFftThreads) / N0));
 }
 
-// Line lengths with compile-time kernels: (L, tile lines of a y / z pass,
-// radices). The tile must be the one finish_axis picks for L. Besides the
-// common smooth lengths (and 320, the 160^3 osf-2 grid), the 3-D grids of
-// 96^3 .. 160^3 images at osf 1.5 and 2: those with a prime factor 7 .. 19
-// and the smooth ones that need four stages (144, 180, 216, 240, 288).
-#define GNUFFT_FIXED_FFT_SIZES(X) \
-  X(96, 32, 8, 4, 3)              \
-  X(128, 32, 8, 8, 2)             \
-  X(160, 32, 8, 4, 5)             \
-  X(192, 32, 8, 8, 3)             \
-  X(256, 16, 8, 8, 4)             \
-  X(156, 32, 4, 3, 13)            \
-  X(168, 32, 8, 3, 7)             \
-  X(204, 32, 4, 3, 17)            \
-  X(208, 32, 8, 2, 13)            \
-  X(224, 32, 8, 4, 7)             \
-  X(228, 32, 4, 3, 19)            \
-  X(272, 16, 8, 2, 17)            \
-  X(304, 16, 8, 2, 19)            \
-  X(320, 16, 8, 8, 5)             \
-  X(144, 32, 4, 4, 3, 3)          \
-  X(180, 32, 4, 5, 3, 3)          \
-  X(216, 32, 8, 3, 3, 3)          \
-  X(240, 32, 4, 4, 5, 3)          \
-  X(288, 16, 8, 4, 3, 3)
-
-// Line lengths with compile-time kernels for the x passes only (their y / z
-// passes use the large tiles).
-#define GNUFFT_FIXED_X_SIZES(X) \
-  X(512, 0, 8, 8, 8)
-
 // L has compile-time kernels (x: of an x pass).
 bool fixed_length(int L, bool x) {
 #define GNUFFT_LENGTH_CASE(LEN, TILE, ...) \
@@ -957,19 +965,21 @@ int x_light(int G0, int lines, int Cg, bool adjoint, int* Q) {
 
 // The light kernel's threads for a y / z pass of `tiles` tiles of kLightStripe lines,
 // or 0 where the full tile (`full` of them) is faster (light over full as above):
-//  - a kernel of the length's own: 0.91 .. 1.41;
+//  - a kernel of the length's own: 0.91 .. 1.02 with 256 threads or more up to two
+//    waves per CU, else 1.02 .. 1.41;
 //  - a prime stage: 1.10 .. 1.34 with more waves than the device holds at once
 //    (525^2, 12 coils: 36.3 and 25.9 us), 0.77 .. 1.00 with fewer (of 256
 //    threads or more; short lines 0.97 .. 1.13);
 //  - others: 512 threads or more 0.72 .. 1.02; 256 threads 0.79 .. 0.98 up to 2048
-//    waves, then 1.11 .. 1.21; 128 threads (short lines) 0.95 .. 1.11 and, from 2048
-//    tiles on, 0.83.
+//    waves, then 1.11 .. 1.21; 128 threads (short lines) 0.95 .. 1.03 up to a tile per
+//    CU, 1.05 .. 1.11 up to 2048 tiles, then 0.83.
 int axis_light(int L, uint64_t full, uint64_t tiles) {
-  if (L > kLightPerThread * 1024 / kLightStripe || full >= kLightBlocks || fixed_length(L, false)) return 0;
+  if (L > kLightPerThread * 1024 / kLightStripe || full >= kLightBlocks) return 0;
   const int nt = light_threads(L * kLightStripe);
   const uint64_t waves = tiles * (uint64_t)(nt / 64);
+  if (fixed_length(L, false)) return nt >= 256 && waves <= 512 ? nt : 0;
   if (prime_radix(L)) return nt >= 256 && waves <= kPrimeWaves ? nt : 0;
-  if (nt == 128) return tiles >= 2048 ? nt : 0;
+  if (nt == 128) return tiles <= 256 || tiles >= 2048 ? nt : 0;
   return nt > 256 || waves <= 2048 ? nt : 0;
 }
 

@@ -62,6 +62,30 @@ def test_same_bits_on_both_sides(case):
     assert torch.equal(torch.view_as_real(fwd[0]), torch.view_as_real(fwd[1]))
 
 
+@pytest.mark.parametrize("img, osf", [((160, 120), 1.5), ((96, 160), 1.5), ((120, 96), 1.5), ((72, 90), 2.0),
+                                      ((128, 150), 1.5), ((128, 128), 1.25), ((64, 64, 16), 1.5), ((48, 40, 120), 1.5)],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_bits_do_not_depend_on_the_coils(img, osf):
+    """Two coils alone take light passes, among 32 full tiles. (144, 180 and 240
+    points: kernels of their own with other stages than by the general order.)"""
+    print("case", img, osf, flush=True)
+    torch, pl, _, _ = _setup(img, osf, 1)
+    pl.set_sens(None, 0)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    rnd = lambda *s: torch.view_as_complex(torch.randn(s + (2,), generator=g, device="cuda"))
+    x, k = rnd(32, *reversed(img)), rnd(32, 700)
+    fwd = [torch.empty((n, 700), dtype=torch.complex64, device="cuda") for n in (2, 32)]
+    adj = [torch.empty((n,) + tuple(reversed(img)), dtype=torch.complex64, device="cuda") for n in (8, 32)]
+    for out, n in zip(fwd, (2, 32)):
+        pl.forward(x[:n].contiguous(), out, n)
+    for out, n in zip(adj, (8, 32)):  # (the spread's groups of eight coils in both)
+        pl.adjoint(k[:n].contiguous(), out, n)
+    torch.cuda.synchronize()
+    assert torch.equal(torch.view_as_real(fwd[0]), torch.view_as_real(fwd[1][:2]))
+    assert torch.equal(torch.view_as_real(adj[0]), torch.view_as_real(adj[1][:8]))
+
+
 @pytest.mark.parametrize("case", [((304, 304), 2.0, 32), ((448, 448), 2.0, 32), ((289, 289), 2.0, 32)],
                          ids=lambda c: "x".join(map(str, c[0])) + "_c%d" % c[2])
 def test_not_slower_than_full_tiles(case):
