@@ -1141,9 +1141,6 @@ int gnufft_plan_create(gnufft_plan* plan, const uint32_t img_dims[3], uint32_t k
     delete p;
     return fail(GNUFFT_ERR_UNSUPPORTED, "plan_create: padded sector width above 255");
   }
-  g.mP = udiv_magic((uint32_t)g.P);
-  g.mP2 = udiv_magic((uint32_t)(g.P * g.P));
-  g.mPD = udiv_magic((uint32_t)(g.dim == 3 ? g.P * g.P * g.P : g.P * g.P));
   g.lookup = lookup;
   const long K = lut_size(osf, kernel_width, lookup);
   if (K < 2 || K > 100000) {

@@ -37,16 +37,12 @@ struct Geom {
   long long Ni;     // image points per coil
   int M;            // samples
   float fft_scale;  // 1/sqrt(Ng)
-  // multiply-high reciprocals: q = umulhi(n, mP) == n / P for n < 2^20
-  uint32_t mP, mP2, mPD;  // for P, P*P and the padded sector point count
 };
 
 // ceil(2^32 / d): exact quotient via __umulhi(n, m) for n*d < 2^32.
 __host__ inline uint32_t udiv_magic(uint32_t d) {
   return (uint32_t)((0x100000000ull + d - 1) / d);
 }
-
-__device__ inline uint32_t udiv(uint32_t n, uint32_t m) { return __umulhi(n, m); }
 
 // One gridding work item: samples [begin, end) of a sector.
 struct Chunk {
@@ -200,22 +196,6 @@ __device__ __host__ inline int round_index(float x) {
 __device__ __host__ inline bool axis_weight(const Geom& g, const float* lut, int a, int i,
                                             int center, float pos, float* w) {
   float kp = map_grid_to_kspace(i, g.G[a], center, g.off);
-  float d = (kp - pos) * g.aniso[a];
-  d *= d;
-  if (g.lookup == 0) {
-    if (!(d < g.rsq)) return false;
-    int li = round_index(d * g.dist_mult);
-    *w = lut[li < g.K - 1 ? li : g.K - 1];
-    return true;
-  }
-  *w = lerp_fetch(lut, g.K, d * g.rsq_inv);
-  return true;
-}
-
-// Same weight with the tap's k-space position precomputed
-// (kp = map_grid_to_kspace(i, G, center, off), identical float value).
-__device__ __host__ inline bool axis_weight_kp(const Geom& g, const float* lut, int a, float kp,
-                                               float pos, float* w) {
   float d = (kp - pos) * g.aniso[a];
   d *= d;
   if (g.lookup == 0) {

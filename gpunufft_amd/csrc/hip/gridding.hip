@@ -82,8 +82,6 @@ void partition_items(const uint32_t* costs, uint32_t n, BatchList* l) {
   l->n = n;
 }
 
-static inline uint32_t batch_blocks(const BatchList& l) { return 8u * (l.max_range ? l.max_range : 1u); }
-
 // ---------------------------------------------------------------------------
 // Interp
 // ---------------------------------------------------------------------------

@@ -18,8 +18,11 @@
 // those that cover it, in a fixed order (periodic wrap and INVERSE fftshift folded
 // in).
 //
-// Bound: the sub-grids' way to memory and back (they hold each point 1.6 times in
-// 2-D and 2 times in 3-D at sector width 8 and kernel width 3) and the LDS atomics.
+// Bound: the LDS atomics, and the sub-grids' way to memory and back (each grid point
+// 1.6 times in 2-D and 2 times in 3-D at sector width 8 and kernel width 3). Per
+// iteration at 525^2, kernel width 3, 12 coils, 122 k samples: sums 81 us, fold 24 us.
+// A thread of the fold takes four coils (with one, ten iterations took 3042 instead
+// of 2929 us).
 
 #include <algorithm>
 
