@@ -3,24 +3,24 @@
 The sector width trades LDS footprint and per-sector fixed costs (the
 interp's staging) against sector occupancy. The best width depends on
 the image size, trajectory density and coil count. For one operator
-shape, best_sector_width builds a plan for every candidate width, times it
-on device-resident data with HIP events, and returns the fastest width. Results are cached per
+shape, best_sector_width builds a plan for every candidate width, times the
+spread (with its reduction) and the interpolation on device-resident
+data with HIP events, and returns the fastest width. Results are cached per
 (image size, kernel width, osf, sample count, coil count) so operators of one
 shape are tuned once.
 
 A batch runs every operator inside launches that fill the GPU, so what an
 operator costs there is its share of a full GPU, not the latency of a lone
 launch (which favours small sectors: more workgroups for a small operator).
-With fill_blocks set (the default), a batch of copies of the operator is
-timed, as many as make about that many workgroups, and the time is divided by
-their number: the coil groups of the kernels follow the operator's own coil
-count, as where it is used.
+With fill_blocks set (the default), the timed launches repeat the coil set
+until they hold about that many workgroups, and the time is divided by the
+repeat count.
 
-Workgroup size and coil groups follow from the width: the interp sizes them
-to the padded sector of the chosen width. For one plan,
-best_workgroups_per_cu then times the gridding at each workgroups-per-CU
-target of the interp (8, 4, 2 or 1 coils of the padded sector in LDS) and
-keeps the fastest on the plan.
+Workgroup size and coil blocking follow from the width: the kernels size
+their LDS rounds and coil blocks to the padded sector of the chosen width.
+For one plan, best_workgroups_per_cu then times the kernel-width-3 gridding
+kernels at each workgroups-per-CU target (the coil block they pick: 4, 2
+or 1 coils of the padded sector in LDS) and keeps the fastest on the plan.
 """
 
 from __future__ import annotations
@@ -33,10 +33,9 @@ _CACHE: dict = {}
 def best_sector_width(img_dims, kernel_width, osf, traj, dens, n_coils, widths=(4, 8, 16),
                       lookup=capi.LOOKUP_NEAREST, reps=3, fill_blocks=4096, max_repeat=16):
     """traj (d, M) / dens (M,) float32 device tensors; returns the width of
-    `widths` with the shortest adjoint + forward time in a batch of copies of
-    the operator (at most max_repeat) that holds about fill_blocks workgroups.
-    fill_blocks=0, or a width that a batch does not take: the spread + interp
-    time of the operator alone."""
+    `widths` with the shortest spread + interp time per coil set, timed with
+    the coil set repeated (at most max_repeat times) until a launch holds
+    about fill_blocks workgroups (fill_blocks=0: the operator alone)."""
     import torch
 
     key = (tuple(img_dims), kernel_width, float(osf), int(traj.shape[1]), int(n_coils),
@@ -56,42 +55,26 @@ def best_sector_width(img_dims, kernel_width, osf, traj, dens, n_coils, widths=(
         if fill_blocks:
             per_set = max(1, info.n_chunks) * -(-n_coils // 8)  # chunks x 8-coil blocks
             rep = max(1, min(max_repeat, -(-fill_blocks // per_set)))
-        shape = tuple(int(x) for x in img_dims)[::-1]
-        batch = None
-        if rep > 1:
-            try:
-                batch = capi.Batch([p] * rep, [n_coils] * rep)
-            except capi.GnufftError:
-                rep = 1  # padded sector too large for the batch kernels
-        k = [torch.zeros((n_coils, M), dtype=torch.complex64, device="cuda") for _ in range(rep)]
-        if batch is not None:
-            x = [torch.zeros((n_coils,) + shape, dtype=torch.complex64, device="cuda") for _ in range(rep)]
-
-            def once():
-                batch.adjoint(k, x)
-                batch.forward(x, k)
-        else:
-            gshape = (n_coils,) + tuple(int(n) for n in info.grid[:len(img_dims)][::-1])
-            grid = torch.empty(gshape, dtype=torch.complex64, device="cuda")
-
-            def once():
-                p.spread_sorted(k[0], grid, n_coils)
-                p.interp_sorted(grid, k[0], n_coils)
-        once()
+        C = n_coils * rep
+        data = torch.zeros((C, M), dtype=torch.complex64, device="cuda")
+        gshape = (C,) + tuple(int(x) for x in info.grid[:len(img_dims)][::-1])
+        grid = torch.empty(gshape, dtype=torch.complex64, device="cuda")
+        out = torch.empty((C, M), dtype=torch.complex64, device="cuda")
+        p.spread_sorted(data, grid, C)
+        p.interp_sorted(grid, out, C)
         ts = []
         for _ in range(reps):
             a = torch.cuda.Event(enable_timing=True)
             b = torch.cuda.Event(enable_timing=True)
             a.record()
-            once()
+            p.spread_sorted(data, grid, C)
+            p.interp_sorted(grid, out, C)
             b.record()
             b.synchronize()
             ts.append(a.elapsed_time(b))
         t = min(ts) / rep
         if best_t is None or t < best_t:
             best, best_t = sw, t
-        if batch is not None:
-            batch.close()
         p.close()
     if best is None:
         raise capi.GnufftError(capi.OK + 5, "no sector width of %s fits this operator" % (widths,))
