@@ -286,8 +286,8 @@ class Plan:
         return grid
 
     def set_workgroups_per_cu(self, n):
-        """Workgroups per CU the kernel-width-3 gridding kernels size their
-        coil block for (0: default)."""
+        """Workgroups per CU the interp sizes its coil groups for (0:
+        default)."""
         check(load().gnufft_plan_set_workgroups_per_cu(self._h, int(n)))
 
     def set_fft(self, kind):
