@@ -1745,7 +1745,7 @@ int gnufft_forward(gnufft_plan p, const void* img, void* out, uint32_t n_coils, 
 // ---------------------------------------------------------------------------
 }  // extern "C"
 
-constexpr int kSpreadNc[3] = {2, 4, 8};  // coil-group sizes of the batched spread
+constexpr int kSpreadNc[4] = {1, 2, 4, 8};  // coil-group sizes of the batched spread
 constexpr int kInterpNc[4] = {1, 2, 4, 8};
 
 struct gnufft_batch_s {
@@ -1758,8 +1758,8 @@ struct gnufft_batch_s {
   BatchOp* ops_d = nullptr;
   uint4* items_d = nullptr;
   // one list per coil-group size (kSpreadNc, kInterpNc)
-  BatchList spread[3]{}, reduce{}, interp[4]{}, post{}, pre{};
-  size_t spread_lds[3] = {0, 0, 0}, interp_lds[4] = {0, 0, 0, 0};
+  BatchList spread[4]{}, reduce{}, interp[4]{}, post{}, pre{};
+  size_t spread_lds[4] = {0, 0, 0, 0}, interp_lds[4] = {0, 0, 0, 0};
   int taps = 3;  // of the interp kernels
   bool full_taps = true;
   float2* grid_d = nullptr;
@@ -1927,8 +1927,8 @@ int gnufft_batch_create(gnufft_batch* batch, const gnufft_plan* plans, uint32_t 
   // descriptors and item lists
   // spread items (tile chunk, coil group) and interp items (chunk, coil group)
   // by group size
-  std::vector<uint4> sp[3], il[4], rd, po, pr;
-  std::vector<uint32_t> sp_cost[3], il_cost[4];
+  std::vector<uint4> sp[4], il[4], rd, po, pr;
+  std::vector<uint32_t> sp_cost[4], il_cost[4];
   for (uint32_t k = 0; k < n_plans && !rc; k++) {
     const gnufft_plan p = b->plans[k];
     const uint32_t C = b->coils[k];
@@ -2029,7 +2029,7 @@ int gnufft_batch_create(gnufft_batch* batch, const gnufft_plan* plans, uint32_t 
       }
       at += v.size();
     };
-    for (int q = 0; q < 3; q++) list(b->spread[q], sp[q], &sp_cost[q]);
+    for (int q = 0; q < 4; q++) list(b->spread[q], sp[q], &sp_cost[q]);
     for (int q = 0; q < 4; q++) list(b->interp[q], il[q], &il_cost[q]);
     list(b->reduce, rd, nullptr);
     list(b->post, po, nullptr);
@@ -2112,7 +2112,7 @@ int gnufft_batch_adjoint(gnufft_batch b, const void* const* kdata, void* const* 
   }
   int rc = batch_upload_ops(b, s);
   if (rc) return rc;
-  for (int q = 0; q < 3; q++)
+  for (int q = 0; q < 4; q++)
     HIP_TRY(launch_spread_batch(b->dim, b->nx == 8 ? 8 : 4, kSpreadNc[q], b->ops_d, b->spread[q], b->spread_lds[q], s));
   HIP_TRY(launch_tile_reduce_batch(b->dim, b->ops_d, b->reduce, s));
   if (b->fused) {

@@ -78,7 +78,7 @@ __host__ __device__ constexpr int tile_subs(int dim) { return dim == 3 ? 8 : 4; 
 // Coils per workgroup of the spread: the block's 16 columns are 8 / NC
 // points in x times NC coils.
 __host__ __device__ constexpr int tile_coils(int n_coils) {
-  return n_coils > 4 ? 8 : n_coils > 2 ? 4 : 2;
+  return n_coils > 4 ? 8 : n_coils > 2 ? 4 : n_coils;
 }
 constexpr uint32_t kNoSlot = ~0u;
 

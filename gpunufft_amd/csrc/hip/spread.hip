@@ -15,7 +15,14 @@
 //   D[row][(x, coil, re/im)] += (wz wy)[row][k] * (wx v)[k][(x, coil, re/im)],
 // run as v_mfma_f32_16x16x4_f32, four samples per instruction: 8 / NC points
 // in x times NC coils fill the 16 columns. Products and sums are 32-bit
-// floats throughout.
+// floats throughout. With one coil a sub-tile is 8 points wide: a matrix
+// instruction covers all of it, where the columns of a second coil would idle.
+// Against the two-coil kernel on one coil, over 48 volumes (64^3..152^3, osf
+// 1.25..2, kernel width 3 and 5, an eighth of the fully sampled spokes to all):
+// 152^3 osf 1.5 width 5 fully sampled 793 -> 545 us (sector sub-grids: 681),
+// 128^3 osf 1.25 width 5 685 -> 495 (458), 128^3 osf 1.5 width 3 306 -> 248
+// (216), 64^3 osf 1.5 width 3 84 -> 82 (54); the geometric mean goes from 0.78
+// to 0.65 of the sector sub-grids' time, the volumes above it from 14 to 6.
 //
 // A tile's samples are taken in rounds of ER: weights (dense over the tile's
 // points per axis) and density-weighted values are staged in LDS once for the
@@ -57,16 +64,18 @@ template <int DIM, int NC>
 struct TileShape {
   static constexpr int TX = tile_width(DIM, 0), TY = tile_width(DIM, 1), TZ = tile_width(DIM, 2);
   static constexpr int SUM = TX + TY + (DIM == 3 ? TZ : 0);
-  static constexpr int SX = 4;                      // x points of a sub-tile
+  static constexpr int SX = NC == 1 ? 8 : 4;        // x points of a sub-tile
   static constexpr int XB = 8 / NC;                 // x points in the 16 columns
   static constexpr int NM = SX / XB;                // 16 x 16 blocks of a sub-tile
   static constexpr int NSX = TX / SX;
-  static constexpr int NW = tile_subs(DIM);
+  static constexpr int NW = tile_subs(DIM) * 4 / SX;
   static constexpr int NT = 64 * NW;
   static constexpr int H = DIM == 3 ? 4 : 2;        // staging threads per sample
   static constexpr int ER = NT / H;                 // samples per round
-  // values: PP threads of two coils (16 bytes) per sample, VI samples each
-  static constexpr int PP = NC / 2;
+  // values: PP threads of two coils (16 bytes) per sample, VI samples each; one
+  // coil: the last threads (in 3-D they have no axis)
+  static constexpr int PP = NC == 1 ? 1 : NC / 2;
+  static constexpr int V0 = NC == 1 ? NT - ER : 0;
   static constexpr int VI = ER * PP > NT ? ER * PP / NT : 1;
   // floats per staged sample: weights per axis, values; a multiple of four
   // with an odd quotient, so rows of different samples start in 16 distinct
@@ -86,7 +95,7 @@ struct TileShape {
   static constexpr size_t staged = list_off + (size_t)NW * ER + 16;
   static constexpr size_t out = (size_t)NC * CS * 4;
   static constexpr size_t lds = staged > out ? staged : out;
-  static_assert(ER == 128, "the threads of a wave share a staging role, a list holds bytes");
+  static_assert(ER % 64 == 0 && ER < 255, "the threads of a wave share a staging role, a list holds bytes");
 };
 
 // Workgroup bid -> work item: runs of kRun consecutive items per XCD
@@ -186,8 +195,8 @@ __device__ __forceinline__ void tile_spread_body(const Geom& g, const SpreadArgs
   const int h = __builtin_amdgcn_readfirstlane(tid / ER);
   const bool has_axis = h < DIM;
   const int axis = has_axis ? h : 0;
-  const int ve = tid / S::PP, part = tid % S::PP;
-  const bool has_value = ve < ER;
+  const int ve = (tid - S::V0) / S::PP, part = tid % S::PP;
+  const bool has_value = tid >= S::V0 && ve < ER;
   const bool dens = a.dens != nullptr;
   const float4* taps = a.taps + (size_t)axis * g.M * (NX / 4);
   const float2* data = a.data + (size_t)(coil0 + 2 * part) * a.coil_stride;
@@ -274,7 +283,7 @@ __device__ __forceinline__ void tile_spread_body(const Geom& g, const SpreadArgs
     for (int q = 0; q < ER / 64; q++) {
       const int s = q * 64 + lane;
       const uint32_t hb = *reinterpret_cast<const uint32_t*>(hit + 4 * s);
-      bool in = (hb >> sx) & 1u;
+      bool in = (hb >> (sx * (S::SX / 4))) & ((1u << (S::SX / 4)) - 1u);
       if (DIM == 3) in = in && ((hb >> (8 + sy)) & 1u);
       const uint64_t b = __ballot(in);
       if (in) {
@@ -303,7 +312,7 @@ __device__ __forceinline__ void tile_spread_body(const Geom& g, const SpreadArgs
         wa[q] = row[q][off_a];
         if (DIM == 3) wa[q] *= row[q][off_z];
         val[q] = row[q][off_v];
-        if constexpr (NC == 8) {
+        if constexpr (NC == 8) {  // (SX == 4)
           const float4 w4 = *reinterpret_cast<const float4*>(row[q] + S::SX * sx);
           wx[q][0] = w4.x, wx[q][1] = w4.y, wx[q][2] = w4.z, wx[q][3] = w4.w;
         } else {
@@ -422,7 +431,8 @@ hipError_t tile_launch_nc(const Geom& g, const SpreadArgs& a, hipStream_t s) {
   switch (tile_coils(a.n_coils)) {
     case 8: return tile_launch<DIM, 8, NX>(g, a, s);
     case 4: return tile_launch<DIM, 4, NX>(g, a, s);
-    default: return tile_launch<DIM, 2, NX>(g, a, s);
+    case 2: return tile_launch<DIM, 2, NX>(g, a, s);
+    default: return tile_launch<DIM, 1, NX>(g, a, s);
   }
 }
 
@@ -483,7 +493,8 @@ hipError_t tile_batch_nc(int nc, const BatchOp* ops, const BatchList& l, size_t 
   switch (nc) {
     case 8: return tile_batch<DIM, 8, NX>(ops, l, lds, s);
     case 4: return tile_batch<DIM, 4, NX>(ops, l, lds, s);
-    default: return tile_batch<DIM, 2, NX>(ops, l, lds, s);
+    case 2: return tile_batch<DIM, 2, NX>(ops, l, lds, s);
+    default: return tile_batch<DIM, 1, NX>(ops, l, lds, s);
   }
 }
 
@@ -510,7 +521,8 @@ size_t spread_lds_bytes(int dim, int nc) {
   switch (nc) {
     case 8: return dim == 3 ? TileShape<3, 8>::lds : TileShape<2, 8>::lds;
     case 4: return dim == 3 ? TileShape<3, 4>::lds : TileShape<2, 4>::lds;
-    default: return dim == 3 ? TileShape<3, 2>::lds : TileShape<2, 2>::lds;
+    case 2: return dim == 3 ? TileShape<3, 2>::lds : TileShape<2, 2>::lds;
+    default: return dim == 3 ? TileShape<3, 1>::lds : TileShape<2, 1>::lds;
   }
 }
 
